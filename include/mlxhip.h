@@ -495,7 +495,9 @@ int mlxhip_cast(const void* x, int32_t src_dtype, void* y, int32_t dst_dtype,
  * values); activations, the KV cache and accumulation are f32. The reference
  * keeps the KV cache in host vectors and re-uploads it every step; here the
  * cache, the token history and the argmax stay on the device and one step is
- * replayed as a HIP graph. Prompt tokens are consumed one position per step.
+ * replayed as a HIP graph. A prompt of three or more tokens is consumed many
+ * positions per pass over the weights, with the results (bit for bit) of a
+ * step per position.
  * Requirements: max_batch <= 8, d_model and hidden multiples of 32,
  * head_dim (d_model / n_heads) one of 8, 16, 32, 64, 128, 256. The captured
  * graph of a (batch, prompt_len[, positions with logits]) shape is kept for

@@ -61,6 +61,7 @@ SOURCES = [
     "kernels/gemm16_x6.hip",
     "kernels/gemm16_small.hip",
     "kernels/decode.hip",
+    "kernels/prefill.hip",
     "kernels/attention.hip",
     "kernels/attention_bwd.hip",
 ]
@@ -68,8 +69,10 @@ SOURCES = [
 
 # Per-source flags. The attention kernel rescales its MFMA accumulators with
 # VALU multiplies every key tile; in the VGPR form of the MFMA instructions
-# they are not copied to and from the accumulation registers for that.
+# they are not copied to and from the accumulation registers for that. The
+# prefill GEMM adds its accumulators up after every k-slice.
 EXTRA = {
+    "kernels/prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "kernels/attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 

@@ -129,6 +129,48 @@ int dec_embed(const uint16_t* emb, const int* tokens, float* x, uint16_t* xs, in
 int dec_finish(const uint64_t* part, int groups, int* tokens, int* argmax_out, const uint16_t* emb, float* x,
                uint16_t* xs, int d, int vocab, int batch, int prompt_len, int* tctr, hipStream_t s);
 int dec_set_counter(int* p, int v, hipStream_t s);
+// The k-slices of a GEMV of this shape: how many, and the width of each.
+void dec_gemv_slices(int n, int k, bool argmax, int* slices, int* width);
+
+// ── prefill.hip (many prompt positions of the decoder at once) ────────────
+// A pass's rows: row b * cp + p is position t0 + p of sequence b. Planes of
+// activations are in MFMA fragment order (as the weights), three of `plane`
+// elements each, rows padded to a multiple of 16. Results have the bits of the
+// one-position step's.
+enum PrefillEpilogue {
+    PREFILL_QKV = 1,     // q -> out [rows][ldo], k / v -> KV cache
+    PREFILL_RESID = 2,   // out[row][n] += y, and its planes (no norm)
+    PREFILL_SILU = 3,    // silu(y) -> planes
+    PREFILL_LOGITS = 4,  // logits[b*ldo + t*n + n'] (may be null) and partial maxima, positions below t_end
+};
+struct PrefillGemm {
+    const uint16_t* w = nullptr;     // fragment-ordered [ceil(N/16)*16][K]
+    const uint16_t* bias = nullptr;  // bf16 [N] (not for LOGITS)
+    const uint16_t* xs = nullptr;    // X planes
+    int64_t plane = 0;
+    const float2* rms = nullptr;     // per row: rms, 1 / rms (QKV, SILU, LOGITS)
+    int n = 0, k = 0, rows = 0, cp = 0, t0 = 0, t_end = 0;
+    float* out = nullptr;
+    int64_t ldo = 0;
+    uint16_t* outs = nullptr;        // RESID / SILU: planes of the output
+    int64_t oplane = 0;
+    float* kc = nullptr;             // QKV: caches as in DecGemv
+    float* vc = nullptr;
+    int dmodel = 0, heads = 0, head_dim = 0, tmax = 0;
+    uint64_t* part = nullptr;        // LOGITS: [prefill_part_groups(n)][rows] maxima
+};
+int prefill_part_groups(int n);
+int prefill_embed(const uint16_t* emb, const int* tokens, float* x, uint16_t* xs, int64_t plane, int d, int vocab,
+                  int batch, int cp, int t0, hipStream_t s);
+int prefill_rms(const float* x, float2* rms, int rows, int d, float eps, hipStream_t s);
+int prefill_gemm(int epi, const PrefillGemm& p, hipStream_t s);
+int prefill_argmax(const uint64_t* part, int groups, int rows, int* argmax_out, int batch, int cp, int t0, int t_end,
+                   hipStream_t s);
+int prefill_attention(const float* q, const float* kc, const float* vc, uint16_t* os, int64_t plane, int batch,
+                      int heads, int hd, int tmax, float scale, int t0, int cp, hipStream_t s);
+// Row p of every sequence (of cp) as the step's x and planes; *tctr = t.
+int prefill_last(const float* px, int cp, int p, float* x, uint16_t* xs, int d, int batch, int* tctr, int t,
+                 hipStream_t s);
 
 // ── attention.hip (fused scaled, masked attention of a batch of heads) ────
 // dh in {16, 32, 64, 128}; any tq, tk >= 1 (keys are streamed in tiles).

@@ -43,6 +43,7 @@
 
 #include "../common.hpp"
 #include "../kernels.hpp"
+#include "decode_common.hpp"
 #include "device_math.hpp"
 
 #pragma clang fp contract(off)
@@ -50,6 +51,7 @@
 namespace mlxhip {
 namespace {
 
+using namespace dec;
 using dev::div_by;
 using dev::shared_divisor;
 using dev::sigmoid_ref;
@@ -60,10 +62,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int WAVE = 64;
-constexpr int KSTEP = 32;                 // k per MFMA
 constexpr int NSTEP = 6;                  // MFMA steps per pass (W and X fragments of a pass held in registers)
-constexpr int TILE_N = 16;                // output features per wave tile
 constexpr int MAX_WAVES = 16;
 constexpr int XN = 4;                     // X units (8 k of 3 planes) per thread per round
 // The LM head's shape: one k-slice per wave over the whole K in one pass (up
@@ -76,22 +75,12 @@ constexpr int XPAD = 8;                   // bf16 padding of each LDS plane row 
 constexpr int XROWS = 3 * DEC_MAX_BATCH;  // hi, mid, lo rows of the batch
 constexpr int WSS_FLOATS = 2 * DEC_MAX_BATCH;  // rms, 1/rms
 
-__device__ inline uint32_t bf16_rne(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return u >> 16;
-}
-__device__ inline float bf16_f32(uint32_t h) { return __uint_as_float(h << 16); }
-
 // Writes v as its hi/mid/lo bf16 terms into the planes of `xs` (row b, column n).
 __device__ inline void store_split(uint16_t* xs, int64_t ld, int b, int64_t n, float v) {
-    const uint32_t h = bf16_rne(v);
-    const float r1 = v - bf16_f32(h);
-    const uint32_t m = bf16_rne(r1);
-    const float r2 = r1 - bf16_f32(m);
-    xs[(int64_t)b * ld + n] = (uint16_t)h;
-    xs[(int64_t)(DEC_MAX_BATCH + b) * ld + n] = (uint16_t)m;
-    xs[(int64_t)(2 * DEC_MAX_BATCH + b) * ld + n] = (uint16_t)bf16_rne(r2);
+    uint16_t t[3];
+    split_terms(v, t);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) xs[(int64_t)(q * DEC_MAX_BATCH + b) * ld + n] = t[q];
 }
 
 // Row b of x (and its planes) = f32 of the bf16 embedding row `src`, 8
@@ -112,30 +101,8 @@ __device__ inline void store_embedding_unit(const uint4 e, float* x, uint16_t* x
 // Maximum over the lanes of a wave that share lane % 8 (one sequence each).
 __device__ inline uint64_t wave_max_u64_by8(uint64_t v) {
 #pragma unroll
-    for (int o = 8; o < WAVE; o <<= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)v, o, WAVE);
-        const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), o, WAVE);
-        const uint64_t w = ((uint64_t)hi << 32) | lo;
-        v = w > v ? w : v;
-    }
+    for (int o = 8; o < WAVE; o <<= 1) v = max_u64(v, shfl_xor_u64(v, o));
     return v;
-}
-
-__device__ inline uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)v, o, WAVE);
-        const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), o, WAVE);
-        const uint64_t w = ((uint64_t)hi << 32) | lo;
-        v = w > v ? w : v;
-    }
-    return v;
-}
-
-// Total order of finite floats as unsigned integers, larger value = larger key.
-__device__ inline uint32_t order_key(float f) {
-    const uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
 // ── the split-activation GEMV ──────────────────────────────────────────────
@@ -394,8 +361,8 @@ __global__ __launch_bounds__((NS > NSTEP ? WIDE_WAVES : MAX_WAVES) * WAVE) void 
             }
         } else {  // DEC_EPI_ARGMAX
             if (valid && p.out) p.out[(int64_t)b * p.ldo + (int64_t)t * N + n] = v;
-            const uint64_t key = valid ? ((uint64_t)order_key(v) << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)n) : 0ull;
-            kmax = key > kmax ? key : kmax;
+            const uint64_t key = valid ? logit_key(v, n) : 0ull;
+            kmax = max_u64(kmax, key);
         }
     }
     if constexpr (EPI == DEC_EPI_ARGMAX) {
@@ -509,13 +476,6 @@ __global__ __launch_bounds__(FIN_BLOCK) void decode_finish_kernel(
 // e_j e^(m_w - m) v_j and divides by l at the end. Two barriers in all.
 constexpr int ATT_BLOCK = 256;
 constexpr int ATT_WAVES = ATT_BLOCK / WAVE;
-
-// v[w] of (v0, v1, v2, v3) by value selects on the bits of w (0 <= w < 4).
-__device__ inline float pick4(int w, float v0, float v1, float v2, float v3) {
-    const float lo = (w & 1) ? v1 : v0;
-    const float hi = (w & 1) ? v3 : v2;
-    return (w & 2) ? hi : lo;
-}
 
 template <int HD>
 __global__ __launch_bounds__(ATT_BLOCK) void decode_attn_kernel(const float* __restrict__ q,
@@ -751,6 +711,12 @@ size_t dec_gemv_lds_bytes(int k, int ks, int r, bool argmax, bool norm) {
     if (argmax) b += (size_t)r * TILE_N * DEC_MAX_BATCH * sizeof(uint64_t);
     if (norm) b += (size_t)DEC_MAX_BATCH * (k / 8) * sizeof(float);      // squares of the X units
     return b;
+}
+
+void dec_gemv_slices(int n, int k, bool argmax, int* slices, int* width) {
+    const GemvShape g = gemv_shape(n, k, argmax, 1);
+    *slices = g.ks;
+    *width = g.kw;
 }
 
 int dec_gemv_groups(int n, int k) { return gemv_shape(n, k, true, DEC_MAX_BATCH).grid; }
