@@ -18,17 +18,23 @@
 // the same correctly rounded quotient as a division for normal values.
 //
 // Layout / launch (CDNA4, wave64): a row is owned by WPR wavefronts (64*WPR
-// lanes). Each lane keeps NV vectors of VEC floats of the row in VGPRs, so
+// lanes). Each lane keeps NV vectors of four floats of the row in VGPRs, so
 // the row is read from HBM once and written once. Lane t of the row reads
-// vector j at element (j*64*WPR + t)*VEC: consecutive lanes touch consecutive
-// 16-byte words (dwordx4, fully coalesced). A 256-thread workgroup holds
-// 4/WPR rows. Rows longer than 64*WPR*NV*VEC fall back to a streaming
-// kernel that re-reads the row (three passes).
+// vector j at element (j*64*WPR + t)*4: consecutive lanes touch consecutive
+// 16-byte words (dwordx4, fully coalesced; rows that start at any 4-byte
+// address, through a buffer descriptor). A 256-thread workgroup holds
+// 4/WPR rows; rows of more than 4096 columns take a workgroup of 8 or 16 waves
+// each. HBM-bound: [1000, 32003] runs softmax / LayerNorm / RMSNorm in 50 us
+// (5.1 TB/s, the rate of a large copy) and their VJPs in 70-76 us, against
+// 128-165 and 165-255 us with the streaming kernel; [4000, 5999] in 34-36 and
+// 49-50 us, against 62-83 and 86-115 us. Rows of more than 32768 columns fall
+// back to the streaming kernel, which re-reads the row (three passes).
 #include "../common.hpp"
 #include "../kernels.hpp"
 #include "device_math.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 
 #pragma clang fp contract(off)
 
@@ -58,10 +64,20 @@ __device__ inline float row_reduce(float v, float* slot, int wave_in_row, int la
     if constexpr (WPR > 1) {
         if (lane == 0) slot[wave_in_row] = v;
         __syncthreads();
-        float r = slot[0];
+        if constexpr (WPR > 4) {
+            // Lane i takes wave i % WPR's value; a butterfly over WPR lanes.
+            v = slot[lane % WPR];
 #pragma unroll
-        for (int w = 1; w < WPR; ++w) r = MAX ? fmaxf(r, slot[w]) : r + slot[w];
-        v = r;
+            for (int o = WPR / 2; o > 0; o >>= 1) {
+                const float u = __shfl_xor(v, o, WAVE);
+                v = MAX ? fmaxf(v, u) : v + u;
+            }
+        } else {
+            float r = slot[0];
+#pragma unroll
+            for (int w = 1; w < WPR; ++w) r = MAX ? fmaxf(r, slot[w]) : r + slot[w];
+            v = r;
+        }
     }
     return v;
 }
@@ -91,10 +107,17 @@ __device__ inline void row_reduce_max_sum(float& m, float& s, float* slot, int w
             slot[2 * wave_in_row + 1] = s;
         }
         __syncthreads();
-        m = slot[0];
-        s = slot[1];
+        if constexpr (WPR > 4) {
+            m = slot[2 * (lane % WPR)];
+            s = slot[2 * (lane % WPR) + 1];
 #pragma unroll
-        for (int w = 1; w < WPR; ++w) merge_max_sum(m, s, slot[2 * w], slot[2 * w + 1]);
+            for (int o = WPR / 2; o > 0; o >>= 1) merge_max_sum(m, s, __shfl_xor(m, o, WAVE), __shfl_xor(s, o, WAVE));
+        } else {
+            m = slot[0];
+            s = slot[1];
+#pragma unroll
+            for (int w = 1; w < WPR; ++w) merge_max_sum(m, s, slot[2 * w], slot[2 * w + 1]);
+        }
     }
 }
 
@@ -139,7 +162,19 @@ __device__ inline void row_reduce_moments(float& n, float& mean, float& m2, floa
             slot[3 * wave_in_row + 2] = m2;
         }
         __syncthreads();
-        if constexpr (EQUAL && (WPR & (WPR - 1)) == 0) {
+        if constexpr (WPR > 4) {
+            n = slot[3 * (lane % WPR)];
+            mean = slot[3 * (lane % WPR) + 1];
+            m2 = slot[3 * (lane % WPR) + 2];
+#pragma unroll
+            for (int o = WPR / 2; o > 0; o >>= 1) {
+                if constexpr (EQUAL)
+                    merge_moments_equal(n, mean, m2, __shfl_xor(mean, o, WAVE), __shfl_xor(m2, o, WAVE));
+                else
+                    merge_moments(n, mean, m2, __shfl_xor(n, o, WAVE), __shfl_xor(mean, o, WAVE),
+                                  __shfl_xor(m2, o, WAVE));
+            }
+        } else if constexpr (EQUAL && (WPR & (WPR - 1)) == 0) {
             // Equal counts in every wave: a pairwise tree (waves 2i and 2i+1,
             // then the pairs) merges equal counts at every level, without
             // the division.
@@ -177,10 +212,7 @@ __device__ inline __amdgpu_buffer_rsrc_t row_rsrc(const float* row, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)row, (short)0, bytes, ROW_BUF_FLAGS);
 }
 
-template <int VEC>
-struct Vec;
-template <>
-struct Vec<4> {
+struct Vec {
     static __device__ inline void load_buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float* d) {
         typedef float f32x4 __attribute__((ext_vector_type(4)));
         const f32x4 t = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, ROW_NT));
@@ -192,7 +224,13 @@ struct Vec<4> {
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{d[0], d[1], d[2], d[3]}), r, off, 0,
                                                ROW_NT);
     }
-    using T = float4;
+    // The n (< 4) values of a row's last vector, each a store of its own.
+    static __device__ inline void store_buf_tail(__amdgpu_buffer_rsrc_t r, uint32_t off, const float* d, int n) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[e]), r,
+                                                  e < n ? off + 4u * (uint32_t)e : ROW_OOB, 0, ROW_NT);
+    }
     // Non-temporal loads: every input element is read exactly once (0.2-0.8
     // us less per [4096, 4096] row op from cold HBM than plain loads).
     static __device__ inline void load(const float* p, float* d) {
@@ -208,35 +246,44 @@ struct Vec<4> {
         __builtin_nontemporal_store(f32x4{d[0], d[1], d[2], d[3]}, reinterpret_cast<f32x4*>(p));
     }
 };
-template <>
-struct Vec<1> {
-    static __device__ inline void load_buf(__amdgpu_buffer_rsrc_t r, uint32_t off, float* d) {
-        d[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, ROW_NT));
-    }
-    static __device__ inline void store_buf(__amdgpu_buffer_rsrc_t r, uint32_t off, const float* d) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d[0]), r, off, 0, ROW_NT);
-    }
-    static __device__ inline void load(const float* p, float* d) { d[0] = __builtin_nontemporal_load(p); }
-    static __device__ inline void store(float* p, const float* d) { __builtin_nontemporal_store(d[0], p); }
-};
+// How a launch's rows fill its vectors: every row exists and holds exactly
+// NV * 4 * 64 * WPR columns; whole vectors, the last ones outside the row; or
+// any number of columns at any 4-byte alignment, where a row's last vector
+// may be partial (the descriptor's range check is per dword: the dwords
+// past the row read as zeros).
+enum RowFill { FILL_EVEN = 0, FILL_VECS = 1, FILL_ANY = 2 };
+
+constexpr int VEC = 4;
+constexpr int row_block(int wpr) { return wpr > 4 ? wpr * WAVE : BLOCK; }
+constexpr bool row_two(int op) { return op == ROW_SOFTMAX_VJP || op == ROW_LAYERNORM_VJP || op == ROW_RMSNORM_VJP; }
+
+// exp(d) for d <= 0 to about an ulp: 2^(d log2 e) with the product's rounding
+// error (and that of the constant) carried to first order.
+__device__ inline float exp_small(float d) {
+    constexpr float L = 1.44269502162933349609375f, L_LO = 1.92596299112661746887e-8f, LN2 = 0.693147182464599609375f;
+    d = d < -200.0f ? -200.0f : d;  // 0 either way; keeps -inf out of the error term and NaN in
+    const float t = d * L;
+    const float e = __builtin_fmaf(d, L_LO, __builtin_fmaf(d, L, -t));
+    const float r = __builtin_amdgcn_exp2f(t);
+    return __builtin_fmaf(r, e * LN2, r);
+}
 
 // a: x (forward) or dy (VJP); b: second operand of a VJP (softmax output s,
-// or the forward input x). p: eps or scale. EVEN: every row of the grid
-// exists and holds exactly NV * VEC * 64 * WPR columns, so no element needs
-// a bounds predicate.
+// or the forward input x). p: eps or scale.
 // Single-input ops are held to 128 VGPRs so four 256-thread workgroups (16
 // waves) are resident per CU: a [4096, 4096] problem is 1024 workgroups, i.e.
 // exactly one round on 256 CUs.
-template <int OP, int WPR, int NV, int VEC, bool EVEN>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
-    (OP == ROW_SOFTMAX_VJP || OP == ROW_LAYERNORM_VJP || OP == ROW_RMSNORM_VJP) ? 2 : 4))) void row_kernel(const float* __restrict__ a,
+template <int OP, int WPR, int NV, int FILL>
+__global__ __launch_bounds__(row_block(WPR)) __attribute__((amdgpu_waves_per_eu(
+    WPR > 4 ? WPR / 4 : row_two(OP) ? 2 : 4))) void row_kernel(const float* __restrict__ a,
                                                     const float* __restrict__ b,
                                                     float* __restrict__ y, int64_t rows,
                                                     int cols, float p, int causal) {
-    constexpr int ROWS_PER_BLOCK = BLOCK / (WAVE * WPR);
+    constexpr bool EVEN = FILL == FILL_EVEN;
+    constexpr int ROWS_PER_BLOCK = row_block(WPR) / (WAVE * WPR);
     constexpr int TPR = WAVE * WPR;  // threads per row
     constexpr int N = NV * VEC;
-    constexpr bool TWO = (OP == ROW_SOFTMAX_VJP || OP == ROW_LAYERNORM_VJP || OP == ROW_RMSNORM_VJP);
+    constexpr bool TWO = row_two(OP);
     // Up to four reductions per kernel, each with its own slots (3 floats per
     // wave for the moment triples).
     __shared__ float red[4][ROWS_PER_BLOCK][WPR > 1 ? 3 * WPR : 1];
@@ -259,7 +306,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
 
     float v[N];
     float w[TWO ? N : 1];
-    bool ok[NV];
+    int have[NV];  // values of vector j inside the row: 0 .. 4
     // Without EVEN, vectors outside the row read as zeros (row_rsrc).
     const int row_bytes = live ? cols * 4 : 0;
     const __amdgpu_buffer_rsrc_t ra = row_rsrc(ar, row_bytes);
@@ -267,16 +314,21 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int c = (j * TPR + t) * VEC;
-        ok[j] = EVEN || (live && c < cols);
+        const bool in = EVEN || (live && c < cols);
+        have[j] = !in ? 0 : FILL == FILL_ANY ? std::min(cols - c, VEC) : VEC;
         if constexpr (EVEN) {
-            Vec<VEC>::load(ar + c, &v[j * VEC]);
-            if constexpr (TWO) Vec<VEC>::load(br + c, &w[j * VEC]);
+            Vec::load(ar + c, &v[j * VEC]);
+            if constexpr (TWO) Vec::load(br + c, &w[j * VEC]);
         } else {
-            const uint32_t off = ok[j] ? 4u * (uint32_t)c : ROW_OOB;
-            Vec<VEC>::load_buf(ra, off, &v[j * VEC]);
-            if constexpr (TWO) Vec<VEC>::load_buf(rb, off, &w[j * VEC]);
+            const uint32_t off = in ? 4u * (uint32_t)c : ROW_OOB;
+            Vec::load_buf(ra, off, &v[j * VEC]);
+            if constexpr (TWO) Vec::load_buf(rb, off, &w[j * VEC]);
         }
     }
+    // Whether vector j is inside the row on every lane (uniform: only the
+    // others' elements are masked one by one), and element e of it here.
+    auto whole = [&](int j) { return EVEN || (j + 1) * TPR * VEC <= cols; };
+    auto has = [&](int j, int e) { return EVEN || (FILL == FILL_ANY ? e < have[j] : have[j] != 0); };
     const float d = (float)cols;
 
     if constexpr (OP == ROW_SOFTMAX || OP == ROW_SCALED_MASKED_SOFTMAX) {
@@ -296,30 +348,38 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
         // exp(x - m_lane) rescaled by exp(m_lane - m_row). exp(d) is
         // 2^(d log2 e) on arguments d <= 0: relative error ~|d| * 2^-24 plus
         // one v_exp_f32 ulp per factor, far inside the 1e-5 tolerance, at a
-        // quarter of expf's VALU cost.
+        // quarter of expf's VALU cost. Rows of 16 waves carry the rounding
+        // errors along (exp_small): as exact as the expf that they had before.
+        constexpr bool LONG = WPR == 16;
         float ml = -INFINITY;
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-            if (ok[j])
+        for (int j = 0; j < NV; ++j) {
+            if (!whole(j))
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) ml = fmaxf(ml, v[j * VEC + e]);
+                for (int e = 0; e < VEC; ++e)
+                    if (!has(j, e)) v[j * VEC + e] = -INFINITY;  // exp 0
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) ml = fmaxf(ml, v[j * VEC + e]);
+        }
+        // A lane whose values are all -inf adds nothing (its exps are 0
+        // against any finite row maximum); a row that is all -inf still ends
+        // as NaN, as exp(-inf - -inf) makes it in the reference.
+        const float mx = ml == -INFINITY ? 0.0f : ml;
         float s = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
 #pragma unroll
             for (int e = 0; e < VEC; ++e) {
-                // A lane whose values are all -inf adds nothing (its exps are
-                // 0 against any finite row maximum); a row that is all -inf
-                // still ends as NaN, as exp(-inf - -inf) makes it in the reference.
-                float ex = (ok[j] && ml != -INFINITY)
-                               ? __builtin_amdgcn_exp2f((v[j * VEC + e] - ml) * 1.44269504088896340736f)
-                               : 0.0f;
+                const float d = v[j * VEC + e] - mx;
+                const float ex = LONG ? exp_small(d) : __builtin_amdgcn_exp2f(d * 1.44269504088896340736f);
                 v[j * VEC + e] = ex;
                 s += ex;
             }
         float m = ml;
         row_reduce_max_sum<WPR>(m, s, slot0, wave_in_row, lane);
-        const float scale = ml == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ml - m) * 1.44269504088896340736f);
+        const float scale = ml == -INFINITY ? 0.0f
+                            : LONG ? exp_small(ml - m)
+                                   : __builtin_amdgcn_exp2f((ml - m) * 1.44269504088896340736f);
         float r;
         row_divisor(s, r);
 #pragma unroll
@@ -331,22 +391,26 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
         float cnt = 0.0f, ls = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            if (ok[j]) {
-                cnt += (float)VEC;
+            if (EVEN || have[j]) {
+                cnt += EVEN ? (float)VEC : (float)have[j];
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) ls += v[j * VEC + e];
+                for (int e = 0; e < VEC; ++e) ls += v[j * VEC + e];  // zeros past the row
             }
         // Whole rows: cnt is N, a power of two, and ls * (1 / N) is ls / N exactly.
         float mean = (EVEN && (N & (N - 1)) == 0) ? ls * (1.0f / (float)N) : (cnt > 0.0f ? ls / cnt : 0.0f);
         float q = 0.0f;
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-            if (ok[j])
+        for (int j = 0; j < NV; ++j) {
+            if (!whole(j))
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    float dv = v[j * VEC + e] - mean;
-                    q += dv * dv;
-                }
+                for (int e = 0; e < VEC; ++e)
+                    if (!has(j, e)) v[j * VEC + e] = mean;  // no deviation
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                float dv = v[j * VEC + e] - mean;
+                q += dv * dv;
+            }
+        }
         row_reduce_moments<WPR, EVEN>(cnt, mean, q, slot0, wave_in_row, lane);
         const float var = q / d;
         float sd = sqrtf(var + p), r;
@@ -379,27 +443,30 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
         const float mean = s / d;
         float q = 0.0f;
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-            if (ok[j])
+        for (int j = 0; j < NV; ++j) {
+            if (!whole(j))
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    float dv = w[j * VEC + e] - mean;
-                    q += dv * dv;
-                }
+                for (int e = 0; e < VEC; ++e)
+                    if (!has(j, e)) w[j * VEC + e] = mean;  // no deviation
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                float dv = w[j * VEC + e] - mean;
+                q += dv * dv;
+            }
+        }
         q = row_reduce<WPR, false>(q, slot1, wave_in_row, lane);
         const float var = q / d;
         const float inv_std = 1.0f / sqrtf(var + p);
         float sdy = 0.0f, sdx = 0.0f;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            if (ok[j])
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    float xh = (w[j * VEC + e] - mean) * inv_std;
-                    w[j * VEC + e] = xh;
-                    sdy += v[j * VEC + e];
-                    sdx += v[j * VEC + e] * xh;
-                }
+            for (int e = 0; e < VEC; ++e) {
+                float xh = (w[j * VEC + e] - mean) * inv_std;
+                w[j * VEC + e] = xh;
+                sdy += v[j * VEC + e];
+                sdx += v[j * VEC + e] * xh;
+            }
         sdy = row_reduce<WPR, false>(sdy, slot2, wave_in_row, lane);
         sdx = row_reduce<WPR, false>(sdx, slot3, wave_in_row, lane);
         const float mdy = sdy / d, mdx = sdx / d;
@@ -428,10 +495,13 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int c = (j * TPR + t) * VEC;
-        if constexpr (EVEN)
-            Vec<VEC>::store(yr + c, &v[j * VEC]);
-        else
-            Vec<VEC>::store_buf(ry, ok[j] ? 4u * (uint32_t)c : ROW_OOB, &v[j * VEC]);
+        if constexpr (EVEN) {
+            Vec::store(yr + c, &v[j * VEC]);
+        } else {
+            Vec::store_buf(ry, have[j] == VEC ? 4u * (uint32_t)c : ROW_OOB, &v[j * VEC]);
+            if (FILL == FILL_ANY && have[j] && have[j] < VEC)
+                Vec::store_buf_tail(ry, 4u * (uint32_t)c, &v[j * VEC], have[j]);
+        }
     }
 }
 
@@ -550,53 +620,49 @@ __global__ __launch_bounds__(BLOCK) void fibre_softmax_kernel(const float* __res
     }
 }
 
-template <int OP, int WPR, int NV, int VEC>
+template <int OP, int WPR, int NV>
 int launch_rows(const float* a, const float* b, float* y, int64_t rows, int64_t cols, float p,
                 int causal, hipStream_t s) {
-    constexpr int RPB = BLOCK / (WAVE * WPR);
-    const int64_t grid = ceil_div(rows, RPB);
-    if (cols == (int64_t)NV * VEC * WAVE * WPR && rows % RPB == 0)
-        hipLaunchKernelGGL((row_kernel<OP, WPR, NV, VEC, true>), dim3((unsigned)grid), dim3(BLOCK), 0,
-                           s, a, b, y, rows, (int)cols, p, causal);
+    constexpr int RPB = row_block(WPR) / (WAVE * WPR);
+    const dim3 grid((unsigned)ceil_div(rows, RPB)), block(row_block(WPR));
+    const uintptr_t at = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(y) |
+                         (row_two(OP) ? reinterpret_cast<uintptr_t>(b) : 0);
+    if (cols % VEC || at % 16)
+        hipLaunchKernelGGL((row_kernel<OP, WPR, NV, FILL_ANY>), grid, block, 0, s, a, b, y, rows, (int)cols, p, causal);
+    else if (cols == (int64_t)NV * VEC * WAVE * WPR && rows % RPB == 0)
+        hipLaunchKernelGGL((row_kernel<OP, WPR, NV, FILL_EVEN>), grid, block, 0, s, a, b, y, rows, (int)cols, p, causal);
     else
-        hipLaunchKernelGGL((row_kernel<OP, WPR, NV, VEC, false>), dim3((unsigned)grid), dim3(BLOCK), 0,
-                           s, a, b, y, rows, (int)cols, p, causal);
+        hipLaunchKernelGGL((row_kernel<OP, WPR, NV, FILL_VECS>), grid, block, 0, s, a, b, y, rows, (int)cols, p, causal);
     return launch_check("row_kernel");
 }
 
 template <int OP>
 int dispatch_rows(const float* a, const float* b, float* y, int64_t rows, int64_t cols, float p,
                   int causal, hipStream_t s, int force_wpr) {
-    const bool two = (OP == ROW_SOFTMAX_VJP || OP == ROW_LAYERNORM_VJP || OP == ROW_RMSNORM_VJP);
-    const bool vec4 = (cols % 4 == 0) && (reinterpret_cast<uintptr_t>(a) % 16 == 0) &&
-                      (reinterpret_cast<uintptr_t>(y) % 16 == 0) &&
-                      (!two || reinterpret_cast<uintptr_t>(b) % 16 == 0);
-    if (vec4) {
-        // force_wpr: 0 = automatic, else waves per row (1, 2 or 4) for tuning.
-        if (force_wpr <= 1) {
-            if (cols <= 256) return launch_rows<OP, 1, 1, 4>(a, b, y, rows, cols, p, causal, s);
-            if (cols <= 512) return launch_rows<OP, 1, 2, 4>(a, b, y, rows, cols, p, causal, s);
-            if (cols <= 1024) return launch_rows<OP, 1, 4, 4>(a, b, y, rows, cols, p, causal, s);
-            if (cols <= 2048) return launch_rows<OP, 1, 8, 4>(a, b, y, rows, cols, p, causal, s);
-        }
-        // 2049..4096 columns: four waves per row (16 values per lane). On
-        // [4096, 4096] with cold HBM this measured 24.3 / 24.0 / 23.4 us for
-        // softmax / LayerNorm / RMSNorm against 25.8 / 24.6 / 24.6 us with one
-        // wave per row and 24.9 / 23.9 / 24.2 us with two: a shorter chain of
-        // arithmetic per wave after its loads land.
-        const int wpr = force_wpr ? force_wpr : 4;
-        if (cols <= 4096) {
-            if (wpr == 1) return launch_rows<OP, 1, 16, 4>(a, b, y, rows, cols, p, causal, s);
-            if (wpr == 2) return launch_rows<OP, 2, 8, 4>(a, b, y, rows, cols, p, causal, s);
-            return launch_rows<OP, 4, 4, 4>(a, b, y, rows, cols, p, causal, s);
-        }
-        if (cols <= 8192) return launch_rows<OP, 4, 8, 4>(a, b, y, rows, cols, p, causal, s);
-        if (cols <= 16384) return launch_rows<OP, 4, 16, 4>(a, b, y, rows, cols, p, causal, s);
-    } else {
-        if (cols <= 256) return launch_rows<OP, 4, 1, 1>(a, b, y, rows, cols, p, causal, s);
-        if (cols <= 1024) return launch_rows<OP, 4, 4, 1>(a, b, y, rows, cols, p, causal, s);
-        if (cols <= 4096) return launch_rows<OP, 4, 16, 1>(a, b, y, rows, cols, p, causal, s);
+    // force_wpr: 0 = automatic, else waves per row (1, 2 or 4) for tuning.
+    if (force_wpr <= 1) {
+        if (cols <= 256) return launch_rows<OP, 1, 1>(a, b, y, rows, cols, p, causal, s);
+        if (cols <= 512) return launch_rows<OP, 1, 2>(a, b, y, rows, cols, p, causal, s);
+        if (cols <= 1024) return launch_rows<OP, 1, 4>(a, b, y, rows, cols, p, causal, s);
+        if (cols <= 2048) return launch_rows<OP, 1, 8>(a, b, y, rows, cols, p, causal, s);
     }
+    // 2049..4096 columns: four waves per row (16 values per lane). On
+    // [4096, 4096] with cold HBM this measured 24.3 / 24.0 / 23.4 us for
+    // softmax / LayerNorm / RMSNorm against 25.8 / 24.6 / 24.6 us with one
+    // wave per row and 24.9 / 23.9 / 24.2 us with two: a shorter chain of
+    // arithmetic per wave after its loads land.
+    const int wpr = force_wpr ? force_wpr : 4;
+    if (cols <= 4096) {
+        if (wpr == 1) return launch_rows<OP, 1, 16>(a, b, y, rows, cols, p, causal, s);
+        if (wpr == 2) return launch_rows<OP, 2, 8>(a, b, y, rows, cols, p, causal, s);
+        return launch_rows<OP, 4, 4>(a, b, y, rows, cols, p, causal, s);
+    }
+    // Longer rows: 16 or 32 values per lane again, over more waves (rows of
+    // 8192 and 16384 columns measured 0.5 us and 3 us less than with four
+    // waves of 32 and 64 values).
+    if (cols <= 8192) return launch_rows<OP, 8, 4>(a, b, y, rows, cols, p, causal, s);
+    if (cols <= 16384) return launch_rows<OP, 16, 4>(a, b, y, rows, cols, p, causal, s);
+    if (cols <= 32768) return launch_rows<OP, 16, 8>(a, b, y, rows, cols, p, causal, s);
     hipLaunchKernelGGL((row_stream_kernel<OP>), dim3((unsigned)rows), dim3(BLOCK), 0, s, a, b, y,
                        rows, cols, p, causal);
     return launch_check("row_stream_kernel");
