@@ -424,14 +424,236 @@ __global__ __launch_bounds__(ATT_THREADS) void attn_fused_kernel(const float* __
 #undef ATT_LOAD
 }
 
+// ── few rows: one workgroup per 16 query rows ──────────────────────────────
+//
+// attn_fused_kernel gives a workgroup two blocks of 64 queries and walks the
+// keys 64 at a time; with few heads and rows most CUs are idle and each
+// busy one works through a chain of iterations (one head of 512 x 512: 4
+// workgroups, 25 us; one query over 2048 keys: one workgroup, 32
+// iterations). Here a workgroup owns 16 query rows and its 8 waves share the
+// keys: wave w takes the 32-key tiles w, w + 8, ... with the same tile
+// arithmetic and a state (m, l, O) of its own, and the eight states are
+// merged through LDS at the end. No tile is used by two waves, so K and V
+// go from memory straight into MFMA operands and are split in registers; no
+// barrier until the merge. Every K and V element is split once per 16 rows
+// instead of once per 64, which is why the other kernel keeps the launches
+// that fill the chip: the splits' VALU operations are what a tile costs here
+// (about 1.5 us with two waves per SIMD).
+constexpr int RB = 16;  // query rows per workgroup
+
+template <int DH>
+__global__ __launch_bounds__(ATT_THREADS) void attn_rows_kernel(const float* __restrict__ q,
+                                                                const float* __restrict__ k,
+                                                                const float* __restrict__ v,
+                                                                float* __restrict__ o, int tq, int tk, int64_t sq,
+                                                                int64_t sk, int64_t sv, int64_t so, float scale,
+                                                                int causal, int nblk, int hg, int rs) {
+    using T = Tile<DH>;
+    constexpr int NS = T::NS, CT = T::CT;
+    constexpr int STATE = 4 * CT + 2;  // O, m, l of one lane
+    __shared__ float merge[ATT_WAVES][STATE][WAVE];
+
+    // A head's blocks on one XCD (its K and V in one L2), the blocks that see
+    // the most keys first.
+    const unsigned L = blockIdx.x, N = gridDim.x;
+    const unsigned logical = N % XCDS == 0 ? (L % XCDS) * (N / XCDS) + L / XCDS : L;
+    const int bh = (int)(logical / (unsigned)nblk), blk = nblk - 1 - (int)(logical % (unsigned)nblk);
+    const int64_t grp = bh / hg, hcol = (int64_t)(bh % hg) * DH;
+    q += grp * sq + hcol;
+    k += grp * sk + hcol;
+    v += grp * sv + hcol;
+    o += grp * so + hcol;
+    const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+    const int li = lane & 15, lg = lane >> 4;
+    const int q0 = blk * RB, row = q0 + li;
+    const int kend = causal ? min(tk, q0 + RB) : tk;
+    const int ntiles = (kend + KT - 1) / KT;
+
+    // Keys of a tile as A operands: half x's lane holds key 16x + li, columns
+    // 32s + 8lg .. +7 (zero past dh). Keys past tk load the last one.
+    float4 kr[2][NS][2];
+    auto load_k = [&](int t) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const float* kp = k + (int64_t)min(t * KT + 16 * x + li, tk - 1) * rs;
+#pragma unroll
+            for (int s = 0; s < NS; ++s)
+                if (DH >= 32 || 8 * lg < DH) {
+                    kr[x][s][0] = *reinterpret_cast<const float4*>(kp + 32 * s + 8 * lg);
+                    kr[x][s][1] = *reinterpret_cast<const float4*>(kp + 32 * s + 8 * lg + 4);
+                }
+        }
+    };
+    auto split8 = [](const float (&x)[8], u32x4 (&out)[3]) {
+        Split3 sp[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sp[e] = split3(x[e]);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            out[0][w] = pack_hi(sp[2 * w].hi, sp[2 * w + 1].hi);
+            out[1][w] = pack_hi(sp[2 * w].mid, sp[2 * w + 1].mid);
+            out[2][w] = pack_hi(sp[2 * w].lo, sp[2 * w + 1].lo);
+        }
+    };
+    // V^T: lane column 16c + li, keys 16x + 4lg + r as k-index 4x + r.
+    float vr[CT][8];
+    auto load_v = [&](int t) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float* vp = v + (int64_t)min(t * KT + 16 * (e >> 2) + 4 * lg + (e & 3), tk - 1) * rs + li;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) vr[c][e] = vp[16 * c];
+        }
+    };
+    if (wave < ntiles) load_k(wave);
+
+    // The query rows as B operands, split.
+    u32x4 qb[NS][3];
+    {
+        const float* qr = q + (int64_t)min(row, tq - 1) * rs;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = 0.0f;
+            if (DH >= 32 || 8 * lg < DH) {
+                const float4 a = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg);
+                const float4 b = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg + 4);
+                x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+            }
+            split8(x, qb[s]);
+        }
+    }
+    float m_run = -INFINITY, l_run = 0.0f;  // of row `row` (the 4 lane groups agree)
+    f32x4 acc[CT];                          // O, columns 16c + 4lg + r
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    for (int t = wave; t < ntiles; t += ATT_WAVES) {
+        load_v(t);
+        // 1. S^T of the two 16-key halves.
+        f32x4 sa[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                float e8[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) e8[e] = 0.0f;
+                if (DH >= 32 || 8 * lg < DH) {
+                    const float4 a = kr[x][s][0], b = kr[x][s][1];
+                    e8[0] = a.x; e8[1] = a.y; e8[2] = a.z; e8[3] = a.w; e8[4] = b.x; e8[5] = b.y; e8[6] = b.z; e8[7] = b.w;
+                }
+                u32x4 ka[3];
+                split8(e8, ka);
+                sa[x] = mma6(ka, qb[s], sa[x]);
+            }
+        if (t + ATT_WAVES < ntiles) load_k(t + ATT_WAVES);
+        float p[2][4];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[x][r] = sa[x][r] * scale;
+        const int kt1 = (t + 1) * KT;
+        if (kt1 > tk || (causal && kt1 - 1 > q0)) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = t * KT + 16 * x + 4 * lg + r;
+                    if (key >= tk || (causal && key > row)) p[x][r] = -INFINITY;
+                    // 0 weight must not meet a non-finite V.
+                    if (key >= tk)
+#pragma unroll
+                        for (int c = 0; c < CT; ++c) vr[c][4 * x + r] = 0.0f;
+                }
+        }
+        // 2. online softmax, as in attn_fused_kernel.
+        float mt = fmaxf(fmaxf(fmaxf(p[0][0], p[0][1]), fmaxf(p[0][2], p[0][3])),
+                         fmaxf(fmaxf(p[1][0], p[1][1]), fmaxf(p[1][2], p[1][3])));
+        mt = lanes_max(mt);
+        const float m_new = fmaxf(m_run, mt);
+        const float m_sub = m_new == -INFINITY ? 0.0f : m_new;
+        const float corr = __builtin_amdgcn_exp2f((m_run - m_sub) * LOG2E);
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) p[x][r] = __builtin_amdgcn_exp2f((p[x][r] - m_sub) * LOG2E);
+        float ps = ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
+        ps = lanes_sum(ps);
+        l_run = l_run * corr + ps;
+        m_run = m_new;
+        // 3. O^T = O^T * corr + V^T P^T.
+        const float pe[8] = {p[0][0], p[0][1], p[0][2], p[0][3], p[1][0], p[1][1], p[1][2], p[1][3]};
+        u32x4 pb[3];
+        split8(pe, pb);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[c][r] *= corr;
+            u32x4 va[3];
+            split8(vr[c], va);
+            acc[c] = mma6(va, pb, acc[c]);
+        }
+    }
+
+    // The waves' states; a wave without a tile left m = -inf, l = 0, O = 0.
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) merge[wave][4 * c + r][lane] = acc[c][r];
+    merge[wave][4 * CT][lane] = m_run;
+    merge[wave][4 * CT + 1][lane] = l_run;
+    __syncthreads();
+    // Wave w merges and stores the columns of c = w, in wave order.
+    static_assert(CT <= ATT_WAVES, "one column tile per wave");
+    if (wave < CT && row < tq) {
+        float m = merge[0][4 * CT][lane];  // finite: tile 0 holds key 0, which every row sees
+#pragma unroll
+        for (int w = 1; w < ATT_WAVES; ++w) m = fmaxf(m, merge[w][4 * CT][lane]);
+        float l = 0.0f, rl;
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < ATT_WAVES; ++w) {
+            const float a = __builtin_amdgcn_exp2f((merge[w][4 * CT][lane] - m) * LOG2E);
+            l += merge[w][4 * CT + 1][lane] * a;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[r] += merge[w][4 * wave + r][lane] * a;
+        }
+        shared_divisor(l, rl);
+        float4 w4;
+        w4.x = div_by(sum[0], l, rl);
+        w4.y = div_by(sum[1], l, rl);
+        w4.z = div_by(sum[2], l, rl);
+        w4.w = div_by(sum[3], l, rl);
+        *reinterpret_cast<float4*>(o + (int64_t)row * rs + 16 * wave + 4 * lg) = w4;
+    }
+}
+
 int64_t blocks_of(int64_t tq) { return (tq + QB - 1) / QB; }
 int64_t pairs_of(int64_t tq) { return (blocks_of(tq) + 1) / 2; }
+
+// Which kernel: measured with both (us, fused / rows), dh 64. Causal 512 x
+// 512: 1 head 25.0 / 10.0, 16 heads 25.4 / 14.4, 32 (1024 workgroups of 16
+// rows) 25.8 / 25.7, 64 25.9 / 48.3; 2048 x 2048, 8 heads (1024) 78.6 / 58.3;
+// 128 x 128, 64 heads (512) 12.0 / 9.3, 128 heads (1024) 12.3 / 16.1; one
+// query over 2048 keys, 1 to 64 heads 73 / 27; 16 queries over 512 keys, 200
+// heads 22 / 12 (the other kernel computes 64 rows however few there are).
+bool few_rows(int64_t batch, int64_t tq, int64_t tk) {
+    return tq <= RB || (tq + RB - 1) / RB * batch <= (tk >= 512 ? 1024 : 640);
+}
 
 template <int DH>
 int launch(const float* q, const float* k, const float* v, float* o, int64_t batch, int64_t tq, int64_t tk,
            int64_t sq, int64_t sk, int64_t sv, int64_t so, float scale, int causal, int hg, int rs,
            hipStream_t s) {
     const int64_t npairs = pairs_of(tq);
+    if (few_rows(batch, tq, tk)) {
+        const int64_t nblk = (tq + RB - 1) / RB;
+        hipLaunchKernelGGL(attn_rows_kernel<DH>, dim3((unsigned)(nblk * batch)), dim3(ATT_THREADS), 0, s, q, k, v, o,
+                           (int)tq, (int)tk, sq, sk, sv, so, scale, causal, (int)nblk, hg, rs);
+        return launch_check("attn_rows_kernel");
+    }
     const dim3 grid((unsigned)(npairs * batch));
     hipLaunchKernelGGL(attn_fused_kernel<DH>, grid, dim3(ATT_THREADS), 0, s, q, k, v, o, (int)tq, (int)tk, sq, sk,
                        sv, so, scale, causal, (int)npairs, (int)blocks_of(tq), hg, rs);
