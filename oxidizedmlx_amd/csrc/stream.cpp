@@ -126,6 +126,80 @@ int64_t tiling_period(const std::vector<int64_t>& src, const std::vector<int64_t
 }  // namespace
 }  // namespace mlxhip
 
+// Whether Concatenate node `id` is multi-head attention written head by head
+// (see HeadConcat in eval); fills its parts. fresh(n): node n is evaluated
+// by this evaluation and not itself asked for.
+template <class Fresh>
+bool mlxhip_stream_t::plan_head_concat(uint64_t id, const Fresh& fresh, uint64_t* src, int64_t* heads,
+                                       std::vector<uint64_t>* inner) {
+    const Node& c = nodes.at(id);
+    const int64_t H = (int64_t)c.inputs.size();
+    if (H < 2 || c.meta.dtype != MLXHIP_DTYPE_F32 || c.meta.shape.size() != 2 ||
+        !(c.op.op.axis == 1 || c.op.op.axis == -1))
+        return false;
+    const Node& first = nodes.at(c.inputs[0]);
+    if (first.op.op.kind != MLXHIP_OP_ATTENTION || first.inputs.size() != 3 || first.meta.shape.size() != 2) return false;
+    const int64_t tq = first.meta.shape[0], dh = first.meta.shape[1];
+    if (c.meta.shape[0] != tq || c.meta.shape[1] != H * dh) return false;
+    uint64_t split[3] = {0, 0, 0};  // the [H, t, dh] Transposes
+    int64_t len[3] = {tq, 0, 0};    // t of Q, K and V
+    for (int64_t i = 0; i < H; ++i) {
+        const uint64_t aid = c.inputs[i];
+        const Node& a = nodes.at(aid);
+        if (!fresh(aid) || consumers[aid] != 1 || a.op.op.kind != MLXHIP_OP_ATTENTION || a.inputs.size() != 3 ||
+            a.meta.dtype != MLXHIP_DTYPE_F32 || a.meta.shape != first.meta.shape ||
+            a.op.op.scale != first.op.op.scale || a.op.op.causal != first.op.op.causal)
+            return false;
+        inner->push_back(aid);
+        for (int j = 0; j < 3; ++j) {
+            const uint64_t rid = a.inputs[j];
+            const Node& r = nodes.at(rid);
+            if (!fresh(rid) || consumers[rid] != 1 || r.op.op.kind != MLXHIP_OP_RESHAPE || r.inputs.size() != 1 ||
+                r.meta.shape.size() != 2)
+                return false;
+            const uint64_t nid = r.inputs[0];
+            const Node& n = nodes.at(nid);
+            if (!fresh(nid) || consumers[nid] != 1 || n.op.op.kind != MLXHIP_OP_NARROW || n.inputs.size() != 1 ||
+                n.op.op.axis != 0 || n.op.op.start != i || n.op.op.length != 1)
+                return false;
+            const uint64_t tid = n.inputs[0];
+            if (i == 0) {
+                const Node& t = nodes.at(tid);
+                const std::vector<int64_t>& ax = t.op.axes;
+                if (!fresh(tid) || consumers[tid] != H || t.op.op.kind != MLXHIP_OP_TRANSPOSE || t.inputs.size() != 1 ||
+                    !t.op.has_axes || ax.size() != 3 || ax[0] != 1 || ax[1] != 0 || ax[2] != 2 ||
+                    t.meta.shape.size() != 3 || t.meta.shape[0] != H || t.meta.shape[2] != dh)
+                    return false;
+                len[j] = t.meta.shape[1];
+                const uint64_t sid = t.inputs[0];
+                const Node& sn = nodes.at(sid);
+                if (sn.op.op.kind != MLXHIP_OP_RESHAPE || sn.inputs.size() != 1 ||
+                    sn.meta.shape != std::vector<int64_t>{len[j], H, dh})
+                    return false;
+                src[j] = sn.inputs[0];
+                const Node& xn = nodes.at(src[j]);
+                if (xn.meta.shape != std::vector<int64_t>{len[j], H * dh}) return false;
+                // A buffer of its own (256-byte aligned), not a view into another's.
+                if (xn.op.op.kind == MLXHIP_OP_NARROW || xn.op.op.kind == MLXHIP_OP_RESHAPE) return false;
+                split[j] = tid;
+                inner->push_back(tid);
+                if (fresh(sid) && consumers[sid] == 1) inner->push_back(sid);
+            } else if (tid != split[j]) {
+                return false;
+            }
+            if (r.meta.shape[0] != len[j] || r.meta.shape[1] != dh ||
+                n.meta.shape != std::vector<int64_t>{1, len[j], dh})
+                return false;
+            inner->push_back(rid);
+            inner->push_back(nid);
+        }
+    }
+    if (split[0] == split[1] || split[0] == split[2] || split[1] == split[2]) return false;
+    if (len[0] != tq || len[1] != len[2] || !attention_fused_supported(dh, tq, len[1])) return false;
+    *heads = H;
+    return true;
+}
+
 int mlxhip_stream_t::eval(const std::vector<uint64_t>& outputs) {
     std::vector<uint64_t> todo;
     for (uint64_t o : outputs) {
@@ -179,6 +253,19 @@ int mlxhip_stream_t::eval(const std::vector<uint64_t>& outputs) {
     std::unordered_map<uint64_t, HeadView> head_in;   // split view node -> where its data lives
     std::unordered_map<uint64_t, HeadView> head_out;  // product -> the merge it writes
     std::unordered_set<uint64_t> head_skip;           // Transposes and inner Reshapes of both
+    // Multi-head attention written head by head (MultiHeadAttention,
+    // crates/mlx-nn/src/attention.rs:47-111): a Concatenate along the columns
+    // of Attention nodes whose operands are Reshape(Narrow(axis 0, i, 1)) of
+    // Transpose{1,0,2}(Reshape [S, H, dh]) of three [S, H*dh] sources. It
+    // runs as one launch that reads the heads side by side in the sources'
+    // rows and writes them so (per head the Attention op's kernel); nothing
+    // in between is materialised.
+    struct HeadConcat {
+        uint64_t src[3];             // the Q, K and V sources
+        std::vector<uint64_t> inner; // every node that it covers, itself apart
+        int64_t H;
+    };
+    std::unordered_map<uint64_t, HeadConcat> head_concat;  // Concatenate -> its heads
     // MLXHIP_HEAD_VIEWS=0: the permutes always run (for comparisons).
     const bool head_views_on = !(getenv("MLXHIP_HEAD_VIEWS") && !strcmp(getenv("MLXHIP_HEAD_VIEWS"), "0"));
     if (fusion) {
@@ -274,6 +361,13 @@ int mlxhip_stream_t::eval(const std::vector<uint64_t>& outputs) {
                 head_in[id] = HeadView{rn.inputs[0], rs[0], rs[1], rs[2], rs[3], t, r};
                 head_skip.insert(t);
                 if (consumers[r] == 1 && fresh(r)) head_skip.insert(r);
+            }
+            for (uint64_t id : order) {
+                if (buffers.count(id) || nodes.at(id).op.op.kind != MLXHIP_OP_CONCATENATE) continue;
+                HeadConcat hc;
+                if (!plan_head_concat(id, fresh, &hc.src[0], &hc.H, &hc.inner)) continue;
+                head_skip.insert(hc.inner.begin(), hc.inner.end());
+                head_concat.emplace(id, std::move(hc));
             }
             // Merges: a rank-3 f32 product (or a Transpose computed as one)
             // whose only reader is Reshape [B, H, S, dh], whose only reader is
@@ -641,12 +735,48 @@ int mlxhip_stream_t::eval(const std::vector<uint64_t>& outputs) {
         *ran = true;
         return MLXHIP_OK;
     };
+    // A Concatenate of attention heads, in one launch from its sources.
+    auto head_attention = [&](uint64_t id, const HeadConcat& hc) -> int {
+        const Node& c = nodes.at(id);
+        mlxhip_input_t ins[3];
+        int64_t shape[3][3];
+        for (int j = 0; j < 3; ++j) {
+            auto b = buffers.find(hc.src[j]);
+            if (b == buffers.end()) return fail(MLXHIP_ERR_INVALID_ARGUMENT, "input node should be evaluated before dependents");
+            const std::vector<int64_t>& s2 = nodes.at(hc.src[j]).meta.shape;
+            shape[j][0] = 1, shape[j][1] = s2[0], shape[j][2] = s2[1];
+            ins[j] = mlxhip_input_t{b->second.ptr, b->second.len, shape[j], 3, MLXHIP_DTYPE_F32};
+        }
+        mlxhip_op_t op = nodes.at(c.inputs[0]).op.c();  // the heads' scale and causal flag
+        op.kind = MLXHIP_OP_HEAD_ATTENTION;
+        op.has_axis = 1;
+        op.axis = (int32_t)hc.H;
+        float* out = nullptr;
+        MLXHIP_TRY(alloc_out(id, &out));
+        const mlxhip_meta_t meta{shape[0], 3, MLXHIP_DTYPE_F32};
+        const int r = eval_node_device(op, ins, 3, meta, out, hs, scratch, nullptr);
+        if (r != MLXHIP_OK) {
+            release_later(out);
+            buffers.erase(id);
+            return r;
+        }
+        eval_calls += 1;
+        launches += 1;
+        for (uint64_t h : hc.inner)
+            if (counted_views.insert(h).second) eval_calls += 1;
+        return MLXHIP_OK;
+    };
     for (size_t oi = 0; oi < order.size(); ++oi) {
         const uint64_t id = order[oi];
         if (buffers.count(id) || folded_transpose.count(id) || interior.count(id) || virtual_bcast.count(id) ||
             absorbed_matmul.count(id) || buffers.count(out_of(id)) ||  // a product already run with its bias term
             head_skip.count(id) || head_in.count(id))                  // head views: read or written in place
             continue;
+        auto hc = head_concat.find(id);
+        if (hc != head_concat.end()) {
+            if ((rc = head_attention(id, hc->second)) != MLXHIP_OK) break;
+            continue;
+        }
         const Node& n = nodes.at(id);
         auto ch = chain_of.find(id);
         auto reads_virtual = [&](const std::vector<uint64_t>& chain) {

@@ -370,6 +370,8 @@ struct mlxhip_stream_t {
         return MLXHIP_OK;
     }
 
+    template <class Fresh>
+    bool plan_head_concat(uint64_t id, const Fresh& fresh, uint64_t* src, int64_t* heads, std::vector<uint64_t>* inner);
     // Evaluates every node in `outputs` (and what they depend on) in one
     // scheduling pass.
     int eval(const std::vector<uint64_t>& outputs);
