@@ -45,6 +45,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
 
 SOURCES = [
     "backend.cpp",
+    "host_copy.cpp",
     "stream.cpp",
     "autograd.cpp",
     "decoder.cpp",

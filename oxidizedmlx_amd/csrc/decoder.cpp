@@ -104,6 +104,10 @@ struct mlxhip_decoder_t {
         graphs.clear();
     }
 
+    mlxhip_decoder_t() { host_copy_retain(); }
+    mlxhip_decoder_t(const mlxhip_decoder_t&) = delete;
+    mlxhip_decoder_t& operator=(const mlxhip_decoder_t&) = delete;
+
     ~mlxhip_decoder_t() {
         (void)hipSetDevice(device);
         if (stream) (void)hipStreamSynchronize(stream);
@@ -114,6 +118,7 @@ struct mlxhip_decoder_t {
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (stream) (void)hipStreamDestroy(stream);
+        host_copy_release();
     }
 
     const uint16_t* lw(int l, int i) const { return w + off_layer[(size_t)l * 8 + i]; }
@@ -600,8 +605,7 @@ int mlxhip_decoder_generate(mlxhip_decoder_t* D, const int32_t* prompt, int32_t 
             for (int t = 0; t < steps; ++t) argmax_out[(size_t)b * steps + t] = am[(size_t)t * batch + b];
     }
     if (want_logits)
-        MLXHIP_HIP(hipMemcpy(logits_out, D->logits, (size_t)batch * steps * c.vocab * sizeof(float),
-                             hipMemcpyDeviceToHost));
+        MLXHIP_TRY(copy_to_host(logits_out, D->logits, (size_t)batch * steps * c.vocab * sizeof(float), s));
     return MLXHIP_OK;
 }
 

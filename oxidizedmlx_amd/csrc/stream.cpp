@@ -1218,8 +1218,9 @@ int mlxhip_stream_get_buffer(mlxhip_stream_t* s, uint64_t node, float* out, size
         return fail_shape({(int64_t)it->second.len}, {(int64_t)len}, "stream_get_buffer");
     if (!len) return MLXHIP_OK;
     MLXHIP_HIP(hipSetDevice(s->device));
-    MLXHIP_HIP(hipMemcpyAsync(out, it->second.ptr, len * sizeof(float), hipMemcpyDeviceToHost, s->hs));
-    return s->drain();
+    const int rc = copy_to_host(out, it->second.ptr, len * sizeof(float), s->hs);
+    const int dr = s->drain();
+    return rc != MLXHIP_OK ? rc : dr;
 }
 
 uint64_t mlxhip_stream_eval_count(const mlxhip_stream_t* s) { return s ? s->eval_calls.load() : 0; }

@@ -117,6 +117,7 @@ struct mlxhip_stream_t {
             return p;
         };
         planes.ctx = this;
+        mlxhip::host_copy_retain();
     }
     mlxhip_stream_t(const mlxhip_stream_t&) = delete;
     mlxhip_stream_t& operator=(const mlxhip_stream_t&) = delete;
@@ -142,6 +143,7 @@ struct mlxhip_stream_t {
         if (join_ev) (void)hipEventDestroy(join_ev);
         if (side) (void)hipStreamDestroy(side);
         if (hs) (void)hipStreamDestroy(hs);
+        mlxhip::host_copy_release();
     }
 
     // The side queue, ready to start after all work queued so far on hs.
