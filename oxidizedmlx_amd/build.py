@@ -53,6 +53,7 @@ SOURCES = [
     "kernels/elementwise.hip",
     "kernels/gemm.hip",
     "kernels/gemm_small.hip",
+    "kernels/gemm_wave.hip",
     "kernels/gemm_thin.hip",
     "kernels/gemm_bf16.hip",
     "kernels/gemm_f16.hip",

@@ -268,12 +268,22 @@ int gemm_thin_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch
                   hipStream_t s);
 
 // gemm_small.hip: f32 products small enough for one or two rounds of 32 x 32
-// tiles with K <= 512, one launch, no workspace, any alignment; operand
-// slices under 2 GiB.
-bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t lda, int64_t ldb, int ta, int tb);
+// tiles, with K <= 128 or in whole aligned tiles with K 256 or 512; one
+// launch, no workspace; operand slices under 2 GiB.
+bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda, int64_t sa,
+                         const float* b, int64_t ldb, int64_t sb, int ta, int tb);
 int gemm_small_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda,
                    int64_t sa, const float* b, int64_t ldb, int64_t sb, float* c, int64_t ldc, int64_t sc,
                    hipStream_t s);
+// gemm_wave.hip: f32 products with few tiles, K split over a workgroup's
+// waves, one launch, no workspace, any alignment; operand slices under 2 GiB.
+// aligned: the other kernels need no packed copies. bias (or null): added to
+// every row of C, one f32 addition to the sum.
+bool gemm_wave_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t lda, int64_t ldb, int ta, int tb,
+                        bool aligned);
+int gemm_wave_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda,
+                  int64_t sa, const float* b, int64_t ldb, int64_t sb, float* c, int64_t ldc, int64_t sc,
+                  const float* bias, hipStream_t s);
 // gemm with the same kernels and plan, its split-K partials and padded
 // operand copies taken from a fixed device array of
 // GEMM_NOALLOC_SCRATCH_BYTES instead of the memory pool: no allocation.

@@ -345,7 +345,7 @@ int fixed_scratch_locked(ScratchState** out) {
 int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
               int64_t batch, const void* a, int64_t lda, int64_t stride_a, const void* b, int64_t ldb,
               int64_t stride_b, void* c, int64_t ldc, int64_t stride_c, hipStream_t s, bool padded,
-              FixedScratch* fs, PlaneCache* cache = nullptr);
+              FixedScratch* fs, PlaneCache* cache = nullptr, const float* bias = nullptr, bool* bias_added = nullptr);
 
 // Generation numbers of split-f32 products: each call's flag value.
 std::atomic<uint32_t> g_x6_gen{0};
@@ -684,9 +684,10 @@ int gemm(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, int64_t
                            s, planes, nullptr, &ran, &bias));
         if (ran) return MLXHIP_OK;
     }
+    bool added = false;
     MLXHIP_TRY(gemm_impl(ab_dtype, c_dtype, trans_a, trans_b, m, n, k, batch, a, lda, stride_a, b, ldb, stride_b, c,
-                         ldc, stride_c, s, false, nullptr, planes));
-    return add_bias(static_cast<float*>(c), m, n, ldc, bias, s);
+                         ldc, stride_c, s, false, nullptr, planes, bias, &added));
+    return added ? MLXHIP_OK : add_bias(static_cast<float*>(c), m, n, ldc, bias, s);
 }
 
 int gemm_noalloc(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
@@ -727,11 +728,12 @@ int gemm_noalloc(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m,
 namespace {
 // padded: the operands are the dispatcher's zero-padded copies (rows
 // readable up to their leading dimension). fs: the fixed scratch of
-// gemm_noalloc, or nullptr to take workspace from the device's pool.
+// gemm_noalloc, or nullptr to take workspace from the device's pool. bias: a
+// row that the kernel adds to C if it can (batch 1, f32); *bias_added says so.
 int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
               int64_t batch, const void* a, int64_t lda, int64_t stride_a, const void* b, int64_t ldb,
               int64_t stride_b, void* c, int64_t ldc, int64_t stride_c, hipStream_t s, bool padded,
-              FixedScratch* fs, PlaneCache* cache) {
+              FixedScratch* fs, PlaneCache* cache, const float* bias, bool* bias_added) {
     if (ab_dtype != MLXHIP_DTYPE_F32 && ab_dtype != MLXHIP_DTYPE_BF16 && ab_dtype != MLXHIP_DTYPE_F16)
         return fail(MLXHIP_ERR_INVALID_ARGUMENT, "gemm: input dtype %d unsupported", ab_dtype);
     if (c_dtype != MLXHIP_DTYPE_F32 && c_dtype != MLXHIP_DTYPE_BF16 && c_dtype != MLXHIP_DTYPE_F16)
@@ -767,28 +769,37 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
         if (ran) return MLXHIP_OK;
     }
 
+    const int ch = 16 / elem_size(ab_dtype);
+    const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
+                         reinterpret_cast<uintptr_t>(b) % 16 == 0 && lda % ch == 0 &&
+                         ldb % ch == 0 && (batch == 1 || (stride_a % ch == 0 && stride_b % ch == 0));
+    const bool direct_f32 = ab_dtype == MLXHIP_DTYPE_F32 && c_dtype == MLXHIP_DTYPE_F32 && gemm_path() == 0;
+    const float* fa = static_cast<const float*>(a);
+    const float* fb = static_cast<const float*>(b);
+
     // Small f32 products (config 1's 512^3): one launch of 32 x 32 tiles with
     // K split across the workgroup's waves, instead of split-K partials and
     // a reduction (measured 13.7 us per call for 512^3 that way, kernels
     // and launches included).
-    if (ab_dtype == MLXHIP_DTYPE_F32 && c_dtype == MLXHIP_DTYPE_F32 && gemm_path() == 0 &&
-        ceil_div(m, 64) * ceil_div(n, 64) * batch < 256 &&
-        gemm_small_f32_fits(m, n, k, batch, lda, ldb, trans_a, trans_b))
-        return gemm_small_f32(trans_a, trans_b, m, n, k, batch, static_cast<const float*>(a), lda, stride_a,
-                              static_cast<const float*>(b), ldb, stride_b, static_cast<float*>(c), ldc, stride_c, s);
+    if (direct_f32 && gemm_small_f32_fits(m, n, k, batch, fa, lda, stride_a, fb, ldb, stride_b, trans_a, trans_b))
+        return gemm_small_f32(trans_a, trans_b, m, n, k, batch, fa, lda, stride_a, fb, ldb, stride_b,
+                              static_cast<float*>(c), ldc, stride_c, s);
 
     // Many f32 products of attention over heads: short-K scores (C = A B^T,
     // bound by writing C) and head-dimension outputs (N = 64, bound by
     // reading A).
     if (ab_dtype == MLXHIP_DTYPE_F32 && c_dtype == MLXHIP_DTYPE_F32 && gemm_path() == 0 &&
         gemm_thin_f32_fits(trans_a, trans_b, m, n, k, batch, a, lda, stride_a, b, ldb, stride_b, c, ldc, stride_c))
-        return gemm_thin_f32(trans_a, trans_b, m, n, k, batch, static_cast<const float*>(a), lda, stride_a,
-                             static_cast<const float*>(b), ldb, stride_b, static_cast<float*>(c), ldc, stride_c, s);
+        return gemm_thin_f32(trans_a, trans_b, m, n, k, batch, fa, lda, stride_a, fb, ldb, stride_b,
+                             static_cast<float*>(c), ldc, stride_c, s);
 
-    const int ch = 16 / elem_size(ab_dtype);
-    const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
-                         reinterpret_cast<uintptr_t>(b) % 16 == 0 && lda % ch == 0 &&
-                         ldb % ch == 0 && (batch == 1 || (stride_a % ch == 0 && stride_b % ch == 0));
+    // Few tiles: K split over the waves of a workgroup, operands straight
+    // into registers at any alignment.
+    if (direct_f32 && !padded && gemm_wave_f32_fits(m, n, k, batch, lda, ldb, trans_a, trans_b, aligned)) {
+        if (bias_added) *bias_added = true;
+        return gemm_wave_f32(trans_a, trans_b, m, n, k, batch, fa, lda, stride_a, fb, ldb, stride_b,
+                             static_cast<float*>(c), ldc, stride_c, bias, s);
+    }
     const int path = gemm_path();
     // 16-bit products the direct-to-LDS kernel cannot read as they are
     // (rows that are not whole 16-byte chunks) or that have too few 128 x 128
@@ -982,7 +993,8 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
     // per workgroup, which on this part writes back the whole L2 of the XCD:
     // measured 4-6x slower.)
     MLXHIP_TRY(run(g, c_dtype));
-    return splitk_reduce(c_dtype, static_cast<const float*>(part), c, m, n, n, ldc, stride_c, g.splits, batch, s);
+    if (bias_added) *bias_added = bias != nullptr;
+    return splitk_reduce(c_dtype, static_cast<const float*>(part), c, m, n, n, ldc, stride_c, g.splits, batch, s, bias);
 }
 }  // namespace
 

@@ -4,8 +4,8 @@
 // C_b[M,N] = op(A_b) * op(B_b), f32 operands and output; replaces matmul
 // (crates/mlx-core/src/cpu_kernels.rs:197-230) at these sizes.
 //
-// One workgroup of 4 waves (one per SIMD) per 32 x 32 tile of C. The K axis
-// is cut into 8 contiguous runs of KH (KH = 8, 16, 32 or 64, the smallest
+// K up to 128: one workgroup of 4 waves (one per SIMD) per 32 x 32 tile of C.
+// The K axis is cut into 8 contiguous runs of KH (KH = 8 or 16, the smallest
 // with 8 * KH >= K), one per half-wave: wave w's half h takes k = (2w + h) *
 // KH + i at MFMA step i of v_mfma_f32_32x32x2_f32, whose two half-waves
 // supply the two k of each step. Each lane thus holds KH consecutive k of
@@ -22,8 +22,8 @@
 // accumulator chains (summed in chain order at the end), so the matrix pipe
 // is not held up by the latency of one chain of dependent MFMAs.
 //
-// Whole-tile products (M, N multiples of 32, K = 8 * KH, every operand run
-// 16-byte aligned) run an 8-wave kernel instead (gemm_small_staged_kernel)
+// Whole-tile products (M, N multiples of 32, K = 64, 128, 256 or 512, every
+// operand run 16-byte aligned) run an 8-wave kernel instead (gemm_small_staged_kernel)
 // that brings MN-contiguous operands in through LDS with 16-byte loads.
 // Measured on MI355X for 512^3 (NN): the 4-wave kernel without range
 // selects took 6.0 us per launch back to back on warm operands (2.5 us of it
@@ -39,7 +39,7 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-constexpr int K_MAX = 512;                   // 8 half-waves x 64 k
+constexpr int K_MAX = 512;                   // 16 half-waves x 32 k (whole tiles)
 constexpr uint32_t OOB_OFF = 0xFFFFFF00u;    // beyond every descriptor range (slices are < 2 GiB)
 constexpr int BUF_FLAGS = 0x00020000;        // gfx9 buffer descriptor word 3 (32-bit data format)
 constexpr int64_t SLICE_MAX_BYTES = int64_t(1) << 31;
@@ -272,43 +272,54 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) void gemm_smal
 // Bytes of one operand slice: `rows` runs of `cols` elements, `ld` apart.
 int64_t slice_bytes(int64_t rows, int64_t cols, int64_t ld) { return ((rows - 1) * ld + cols) * 4; }
 
-template <int TA, int TB, int KH>
-int launch_kh(const SmallArgs& g, bool even, int64_t batch, hipStream_t s) {
-    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)batch);
-    if (even) hipLaunchKernelGGL((gemm_small_staged_kernel<TA, TB, KH / 2>), grid, dim3(512), 0, s, g);
-    else hipLaunchKernelGGL((gemm_small_kernel<TA, TB, KH>), grid, dim3(256), 0, s, g);
-    return launch_check("gemm_small_kernel");
+// Every operand run 16-byte aligned: 16-byte loads along K (K-contiguous
+// operands) or along M / N (the staged, MN-contiguous ones).
+bool staged(int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda, int64_t sa, const float* b,
+            int64_t ldb, int64_t sb) {
+    auto whole = [&](const float* p, int64_t ld, int64_t st) {
+        return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && (batch == 1 || st % 4 == 0);
+    };
+    return m % 32 == 0 && n % 32 == 0 && (k == 64 || k == 128 || k == 256 || k == 512) && whole(a, lda, sa) &&
+           whole(b, ldb, sb);
 }
 
 template <int TA, int TB>
 int launch_small(SmallArgs& g, const float* a, int64_t lda, int64_t sa, const float* b, int64_t ldb, int64_t sb,
                  int64_t batch, hipStream_t s) {
-    const int64_t m = g.m, n = g.n, k = g.k;
-    // k per half-wave: the smallest of 8, 16, 32, 64 covering K in 8 runs.
-    const int kh = k <= 64 ? 8 : k <= 128 ? 16 : k <= 256 ? 32 : 64;
-    // 16-byte loads need every K-contiguous run 16-byte aligned.
-    auto kc_aligned = [&](const float* p, int64_t ld, int64_t st) {
-        return reinterpret_cast<uintptr_t>(p) % 16 == 0 && ld % 4 == 0 && (batch == 1 || st % 4 == 0);
-    };
-    // Whole tiles: 16-byte loads along K (K-contiguous operands) or along
-    // M / N (the staged, MN-contiguous ones) need every run 16-byte aligned.
-    const bool even = m % 32 == 0 && n % 32 == 0 && k == 8 * kh && kc_aligned(a, lda, sa) && kc_aligned(b, ldb, sb);
-    switch (kh) {
-        case 8: return launch_kh<TA, TB, 8>(g, even, batch, s);
-        case 16: return launch_kh<TA, TB, 16>(g, even, batch, s);
-        case 32: return launch_kh<TA, TB, 32>(g, even, batch, s);
-        default: return launch_kh<TA, TB, 64>(g, even, batch, s);
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)batch);
+    if (staged(g.m, g.n, g.k, batch, a, lda, sa, b, ldb, sb)) {
+        switch (g.k) {
+            case 64: hipLaunchKernelGGL((gemm_small_staged_kernel<TA, TB, 4>), grid, dim3(512), 0, s, g); break;
+            case 128: hipLaunchKernelGGL((gemm_small_staged_kernel<TA, TB, 8>), grid, dim3(512), 0, s, g); break;
+            case 256: hipLaunchKernelGGL((gemm_small_staged_kernel<TA, TB, 16>), grid, dim3(512), 0, s, g); break;
+            default: hipLaunchKernelGGL((gemm_small_staged_kernel<TA, TB, 32>), grid, dim3(512), 0, s, g); break;
+        }
+    } else if (g.k <= 64) {
+        hipLaunchKernelGGL((gemm_small_kernel<TA, TB, 8>), grid, dim3(256), 0, s, g);
+    } else {
+        hipLaunchKernelGGL((gemm_small_kernel<TA, TB, 16>), grid, dim3(256), 0, s, g);
     }
+    return launch_check("gemm_small_kernel");
 }
 
 }  // namespace
 
-bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t lda, int64_t ldb, int ta, int tb) {
+bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda, int64_t sa,
+                         const float* b, int64_t ldb, int64_t sb, int ta, int tb) {
     // At most two rounds of 32 x 32 tiles on 256 CUs: beyond that the 64 x 64
     // and larger tiles of the general kernel reuse operands better. Every
     // operand slice must be addressable with 32-bit offsets.
-    if (!(m >= 1 && n >= 1 && k >= 1 && k <= K_MAX && ceil_div(m, 32) * ceil_div(n, 32) * batch <= 512 &&
-          batch <= 65535))
+    if (!(m >= 1 && n >= 1 && k >= 1 && k <= K_MAX && ceil_div(m, 64) * ceil_div(n, 64) * batch < 256 &&
+          ceil_div(m, 32) * ceil_div(n, 32) * batch <= 512 && batch <= 65535))
+        return false;
+    // Other products over a K above 128 are faster in gemm_wave.hip, which
+    // has 16-wide tiles too: 300 x 300 x 500 15.0 us here and 5.5 there. Up to
+    // 128 it is no faster (700 x 700 x 100: 7.0 and 6.9 us) and sums in longer
+    // chains (256 x 100 x 64: error 7.1e-8 here, 8.5e-8 there). Whole tiles,
+    // which run staged, are faster here (512^3 6.3 and 7.1 us) but below 192
+    // of them with K over 256 (256 x 512 x 512: 6.7 and 5.9 us).
+    if (!(k <= 128 || (staged(m, n, k, batch, a, lda, sa, b, ldb, sb) &&
+                       (k <= 256 || (m / 32) * (n / 32) * batch >= 192))))
         return false;
     const int64_t a_bytes = ta ? slice_bytes(k, m, lda) : slice_bytes(m, k, lda);
     const int64_t b_bytes = tb ? slice_bytes(n, k, ldb) : slice_bytes(k, n, ldb);
@@ -319,7 +330,7 @@ bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t
 int gemm_small_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda,
                    int64_t sa, const float* b, int64_t ldb, int64_t sb, float* c, int64_t ldc, int64_t sc,
                    hipStream_t s) {
-    if (!gemm_small_f32_fits(m, n, k, batch, lda, ldb, ta, tb))
+    if (!gemm_small_f32_fits(m, n, k, batch, a, lda, sa, b, ldb, sb, ta, tb))
         return fail(MLXHIP_ERR_INVALID_ARGUMENT, "gemm_small_f32: shape outside the small kernel's range");
     SmallArgs g;
     g.a = a, g.b = b, g.c = c;
