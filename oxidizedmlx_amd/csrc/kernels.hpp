@@ -275,15 +275,16 @@ bool gemm_small_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, const f
 int gemm_small_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda,
                    int64_t sa, const float* b, int64_t ldb, int64_t sb, float* c, int64_t ldc, int64_t sc,
                    hipStream_t s);
-// gemm_wave.hip: f32 products with few tiles, K split over a workgroup's
-// waves, one launch, no workspace, any alignment; operand slices under 2 GiB.
-// aligned: the other kernels need no packed copies. bias (or null): added to
-// every row of C, one f32 addition to the sum.
-bool gemm_wave_f32_fits(int64_t m, int64_t n, int64_t k, int64_t batch, int64_t lda, int64_t ldb, int ta, int tb,
-                        bool aligned);
-int gemm_wave_f32(int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const float* a, int64_t lda,
-                  int64_t sa, const float* b, int64_t ldb, int64_t sb, float* c, int64_t ldc, int64_t sc,
-                  const float* bias, hipStream_t s);
+// gemm_wave.hip: products with few tiles, K split over a workgroup's waves,
+// one launch, no workspace, any alignment; operand slices under 2 GiB; C in
+// f32, bf16 or f16 (f32 for f32 operands). aligned: the other kernels need no
+// packed copies. bias (or null): added to every row of an f32 C, one f32
+// addition to the sum.
+bool gemm_wave_fits(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch, int64_t lda, int64_t ldb, int ta,
+                    int tb, bool aligned);
+int gemm_wave(int ab_dtype, int c_dtype, int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const void* a,
+              int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb, void* c, int64_t ldc, int64_t sc,
+              const float* bias, bool aligned, hipStream_t s);
 // gemm with the same kernels and plan, its split-K partials and padded
 // operand copies taken from a fixed device array of
 // GEMM_NOALLOC_SCRATCH_BYTES instead of the memory pool: no allocation.

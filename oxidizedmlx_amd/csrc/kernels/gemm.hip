@@ -795,10 +795,11 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
 
     // Few tiles: K split over the waves of a workgroup, operands straight
     // into registers at any alignment.
-    if (direct_f32 && !padded && gemm_wave_f32_fits(m, n, k, batch, lda, ldb, trans_a, trans_b, aligned)) {
-        if (bias_added) *bias_added = true;
-        return gemm_wave_f32(trans_a, trans_b, m, n, k, batch, fa, lda, stride_a, fb, ldb, stride_b,
-                             static_cast<float*>(c), ldc, stride_c, bias, s);
+    if ((direct_f32 || (ab_dtype != MLXHIP_DTYPE_F32 && gemm_path() == 0)) && !padded &&
+        gemm_wave_fits(ab_dtype, m, n, k, batch, lda, ldb, trans_a, trans_b, aligned)) {
+        if (bias_added) *bias_added = bias != nullptr;
+        return gemm_wave(ab_dtype, c_dtype, trans_a, trans_b, m, n, k, batch, a, lda, stride_a, b, ldb, stride_b, c,
+                         ldc, stride_c, bias, aligned, s);
     }
     const int path = gemm_path();
     // 16-bit products the direct-to-LDS kernel cannot read as they are

@@ -1,7 +1,7 @@
-"""f32 products with K split over a workgroup's waves (kernels/gemm_wave.hip):
+"""Products with K split over a workgroup's waves (kernels/gemm_wave.hip):
 every tile shape, tile edges and K remainders in all four layouts, gaps
-between rows and slices filled with NaN, operands at any 4-byte alignment,
-against float64 within the f32 summation bound."""
+between rows and slices filled with NaN, operands at any alignment of their
+elements, against float64 within the f32 summation bound."""
 import numpy as np
 import pytest
 
@@ -24,13 +24,13 @@ CASES = [
 ]
 
 
-def embed(rows, offset, gap, slice_gap):
-    """A NaN-filled flat array with the batch's matrices in it: row pitch cols
-    + gap, slices slice_gap apart, starting `offset` floats in."""
+def embed(rows, offset, gap, slice_gap, fill=np.nan):
+    """A flat array of `fill` with the batch's matrices in it: row pitch cols
+    + gap, slices slice_gap apart, starting `offset` elements in."""
     b, r, c = rows.shape
     ld = c + gap
     stride = r * ld + slice_gap
-    buf = np.full(offset + b * stride, np.nan, np.float32)
+    buf = np.full(offset + b * stride, fill, rows.dtype)
     for i in range(b):
         view = buf[offset + i * stride:offset + i * stride + r * ld].reshape(r, ld)
         view[:, :c] = rows[i]
@@ -77,3 +77,42 @@ def test_bias_in_the_store_is_the_separate_addition(rows, inputs, outputs):
     bound = (inputs + 1) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w.T) + np.abs(b)) * 1.01
     for y in res:
         assert (np.abs(y - exact) <= bound).all()
+
+
+CASES16 = [
+    # 16 x 16, 16 x 32, 32 x 32, 32 x 64 and 64 x 64 tiles; rounds of 16-wide
+    # ones for few rows; the last is past the rule.
+    (1, 1, 1, 1), (17, 33, 63, 1), (15, 250, 1601, 1), (33, 31, 217, 50), (8, 4096, 1535, 1),
+    (129, 500, 199, 1), (100, 1500, 65, 1), (5, 30001, 70, 1),
+    (511, 512, 145, 1), (129, 257, 255, 4),
+    (500, 1000, 777, 1), (1000, 1016, 528, 1), (900, 1000, 1023, 1),
+]
+
+
+@pytest.mark.parametrize("m,n,k,batch", CASES16)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("dtype", ["bf16", "f16"])
+def test_16_bit_tiles_remainders_and_gaps(m, n, k, batch, ta, tb, dtype):
+    dt = abi.BF16 if dtype == "bf16" else abi.F16
+    nan16 = 0x7FC0 if dt == abi.BF16 else 0x7E00
+    bits = synth.bf16_bits if dt == abi.BF16 else synth.f16_bits
+    wide = synth.bf16_to_f32 if dt == abi.BF16 else lambda x: x.view(np.float16).astype(np.float32)
+    odd = (m + n + k) % 2
+    a = bits(synth.normal(m + k, (batch, m, k)))
+    b = bits(synth.normal(n + k + 1, (batch, k, n)))
+    fa, lda, stra = embed(np.ascontiguousarray(a.transpose(0, 2, 1)) if ta else a, 3 * odd, 5 * odd, 6 * odd, nan16)
+    fb, ldb, strb = embed(np.ascontiguousarray(b.transpose(0, 2, 1)) if tb else b, odd, 2 * odd, 3 * odd, nan16)
+    da, db = hb.DeviceBuffer.from_array(fa), hb.DeviceBuffer.from_array(fb)
+    exact = {i: (wide(a[i]), wide(b[i])) for i in {0, batch - 1}}
+    for ct in (abi.F32, dt):
+        ldc = n + 3
+        c0 = np.full((batch, m, ldc), 7 if ct == dt else 7.0, np.uint16 if ct == dt else np.float32)
+        dc = hb.DeviceBuffer.from_array(c0)
+        hb.gemm(dt, ct, bool(ta), bool(tb), m, n, k, da.ptr + 6 * odd, lda, db.ptr + 2 * odd, ldb, dc, ldc,
+                batch=batch, stride_a=stra, stride_b=strb, stride_c=m * ldc)
+        hb.synchronize()
+        got = dc.download(c0.dtype).reshape(batch, m, ldc)
+        assert (got[:, :, n:] == 7).all()
+        for i, (x, y) in exact.items():
+            c = got[i, :, :n] if ct == abi.F32 else wide(np.ascontiguousarray(got[i, :, :n]))
+            gemm_full_check(c, x, y, out="f32" if ct == abi.F32 else dtype, what=f"{m}x{n}x{k} {dtype} slice {i}")
