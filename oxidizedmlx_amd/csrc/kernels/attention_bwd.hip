@@ -11,7 +11,8 @@
 //   P_ij = exp(S_ij - L_i),  dP = dO V^T,  dS = P o (dP - D)
 //   dQ = scale * dS K,  dK = scale * dS^T Q,  dV = P^T dO.
 // Nothing of size T x T is stored: two kernels stream over blocks of 64
-// keys (queries) and recompute S and P in registers.
+// keys (queries) and recompute S and P in registers. Scores and L are kept in
+// log2 units (one rounding between S and the exponential).
 //
 //   attn_bwd_dq_kernel, one workgroup per (head, block of 64 queries): a
 //   first pass over the visible key blocks computes L (running max and sum
@@ -20,7 +21,10 @@
 //   attn_bwd_dkdv_kernel, one workgroup per (head, block of 64 keys): over
 //   the query blocks that see them, recomputes P and dS from L and D and
 //   accumulates dK and dV.
+//   With few heads both are sliced over more workgroups (attention_vjp).
 //
+// Bound by the f32 matrix rate (64 heads x 1024, causal: 36.5 GFLOP over the
+// visible blocks in 327 us, 112 TFLOP/s; a large f32 product reaches 138).
 // Products are v_mfma_f32_32x32x2_f32 (exact f32 products, f32 sums). A
 // workgroup's 4 waves each own a 32 x 32 tile of the 64 x 64 block: wave w
 // takes query half qh = w & 1 and key half kh = w >> 1. For an MFMA lane l,
@@ -55,6 +59,7 @@ constexpr int BT = 64;        // queries / keys per block
 constexpr int DH = 64;        // head dimension
 constexpr int PITCH = DH + 4; // LDS row pitch in floats: 16-byte rows, consecutive rows 4 banks apart
 constexpr int THREADS = 4 * WAVE;
+constexpr int64_t CUS = 256;
 constexpr float LOG2E = 1.44269504088896340736f;
 
 __device__ inline int crow(int v, int h) { return 8 * (v >> 2) + 4 * h + (v & 3); }
@@ -142,14 +147,28 @@ __device__ inline void block_of(int id, int heads, int nb, bool heavy_high, int*
     *blk = heavy_high ? b : nb - 1 - b;
 }
 
+// Sliced calls: ck blocks of the sum to a workgroup, n slices at most. ml:
+// [n][rows][2], part: [dQ, dK, dV][n][rows][DH]; rows = heads * T.
+struct Slices {
+    int ck, n;
+    int64_t rows;
+    float* ml;
+    float* part;
+};
+
 // ── dQ, L, D ───────────────────────────────────────────────────────────────
 // S^T tile = K Q^T (rows keys, columns queries): the lane's column is query
-// q = qb*64 + 32 qh + c, so L_q and D_q are per-lane scalars.
+// q = qb*64 + 32 qh + c, so L_q and D_q are per-lane scalars. L is kept in
+// log2 units. WHOLE: both passes over every visible key block. Sliced
+// (blockIdx.y = slice of ck key blocks): LSE makes the slice's (m, l) pairs
+// and D, DQ combines the slices' pairs in order and makes a partial dQ.
+enum Pass { WHOLE, LSE, DQ };
+template <int PASS>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dq_kernel(const float* __restrict__ Q, const float* __restrict__ K,
                                                                const float* __restrict__ V, const float* __restrict__ O,
                                                                const float* __restrict__ dO, float* __restrict__ dQ,
                                                                float* __restrict__ lse_out, float* __restrict__ d_out,
-                                                               int T, float scale, int causal, int hg, int rs) {
+                                                               int T, float scale, int causal, int hg, int rs, Slices slc) {
     // K and V blocks; at the end the kh = 1 partials of dQ ([qh][64 d][33]).
     __shared__ __align__(16) float smem[2 * BT * PITCH];
     __shared__ float xch[2][2][32][2];  // (m, l) per query half, key half, query
@@ -158,6 +177,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int nqb = T / BT;
     int head_i, qb;
     block_of((int)blockIdx.x, (int)(gridDim.x / nqb), nqb, true, &head_i, &qb);
+    int kb0 = 0, nkb = causal ? qb + 1 : nqb;
+    const int slices = PASS == WHOLE ? 1 : (nkb + slc.ck - 1) / slc.ck;
+    if constexpr (PASS != WHOLE) {
+        kb0 = (int)blockIdx.y * slc.ck;
+        if (kb0 >= nkb) return;
+        nkb = min(nkb, kb0 + slc.ck);
+    }
+    const float sl = scale * LOG2E;  // scores in log2 units
     const int64_t head = head_i;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
     const int qh = wave & 1, kh = wave >> 1, c = lane & 31, h = lane >> 5;
@@ -168,8 +195,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     float qr[32], dor[32];
     load_row_half(Qh, q, rs, h, qr);
     load_row_half(dOh, q, rs, h, dor);
+    const int64_t row = head * T + q;
     float Dq;
-    {
+    if constexpr (PASS == DQ) {
+        Dq = d_out[row];
+    } else {
         float orow[32];
         load_row_half(Oh, q, rs, h, orow);
         float s = 0.0f;
@@ -177,7 +207,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int i = 0; i < 32; ++i) s += dor[i] * orow[i];
         Dq = s + __shfl_xor(s, 32, WAVE);
     }
-    const int nkb = causal ? qb + 1 : nqb;
     f32x4 kc[4], vc[4];
 
     // Pass 1: L_q. Lanes c and c + 32 see different key rows of the same
@@ -188,66 +217,83 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // one computes while the other waits for its loads (registers for a
     // prefetch would leave room for only one).
     float m = -INFINITY, l = 0.0f;
-    for (int kb = 0; kb < nkb; ++kb) {
-        block_load(Kh, kb * BT, rs, tid, kc);
-        __syncthreads();  // the previous block's readers are done
-        block_store(Ks, tid, kc);
-        __syncthreads();
-        // Two independent accumulator chains (step s feeds chain s % 2),
-        // summed in chain order: one chain of dependent MFMAs runs at about
-        // half the matrix pipe's rate. Pass 2 sums S the same way.
-        f32x16 s2[2] = {zero16(), zero16()};
-        float kr[32];
-        lds_row32(Ks + (32 * kh + c) * PITCH + 32 * h, kr);
-        __builtin_amdgcn_sched_barrier(0);
+    if constexpr (PASS != DQ) {
+        for (int kb = kb0; kb < nkb; ++kb) {
+            block_load(Kh, kb * BT, rs, tid, kc);
+            __syncthreads();  // the previous block's readers are done
+            block_store(Ks, tid, kc);
+            __syncthreads();
+            // Two independent accumulator chains (step s feeds chain s % 2),
+            // summed in chain order: one chain of dependent MFMAs runs at about
+            // half the matrix pipe's rate. Pass 2 sums S the same way.
+            f32x16 s2[2] = {zero16(), zero16()};
+            float kr[32];
+            lds_row32(Ks + (32 * kh + c) * PITCH + 32 * h, kr);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 32; ++s) mfma(kr[s], qr[s], s2[s & 1]);
-        const f32x16 sa = s2[0] + s2[1];
-        float x[16], mt = -INFINITY;
+            for (int s = 0; s < 32; ++s) mfma(kr[s], qr[s], s2[s & 1]);
+            const f32x16 sa = s2[0] + s2[1];
+            float x[16], mt = -INFINITY;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int key = kb * BT + 32 * kh + crow(v, h);
-            x[v] = (causal && key > q) ? -INFINITY : sa[v] * scale;
-            mt = fmaxf(mt, x[v]);
+            for (int v = 0; v < 16; ++v) x[v] = sa[v] * sl;
+            if (causal && kb == qb) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) x[v] = 32 * kh + crow(v, h) > 32 * qh + c ? -INFINITY : x[v];
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mt = fmaxf(mt, x[v]);
+            const float mn = fmaxf(m, mt);
+            if (mn != -INFINITY) {
+                float acc = 0.0f;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc += exp2_small(x[v] - mn);
+                l = l * exp2_small(m - mn) + acc;
+                m = mn;
+            }
         }
-        const float mn = fmaxf(m, mt);
-        if (mn != -INFINITY) {
-            float acc = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc += exp2_small((x[v] - mn) * LOG2E);
-            l = l * exp2_small((m - mn) * LOG2E) + acc;
+        {
+            const float m2 = __shfl_xor(m, 32, WAVE), l2 = __shfl_xor(l, 32, WAVE);
+            const float mn = fmaxf(m, m2);
+            l = (m == -INFINITY ? 0.0f : l * exp2_small(m - mn)) +
+                (m2 == -INFINITY ? 0.0f : l2 * exp2_small(m2 - mn));
+            m = mn;
+        }
+        if (h == 0) {
+            xch[qh][kh][c][0] = m;
+            xch[qh][kh][c][1] = l;
+        }
+        __syncthreads();
+        {
+            const float m0 = xch[qh][0][c][0], l0 = xch[qh][0][c][1];
+            const float m1 = xch[qh][1][c][0], l1 = xch[qh][1][c][1];
+            const float mn = fmaxf(m0, m1);
+            l = (m0 == -INFINITY ? 0.0f : l0 * exp2_small(m0 - mn)) +
+                (m1 == -INFINITY ? 0.0f : l1 * exp2_small(m1 - mn));
+            m = mn;
+        }
+        if (kh == 0 && h == 0) {
+            if ((int)blockIdx.y == 0) d_out[row] = Dq;
+            if constexpr (PASS == LSE) {
+                float* ml = slc.ml + ((int64_t)blockIdx.y * slc.rows + row) * 2;
+                ml[0] = m, ml[1] = l;
+            }
+        }
+    } else {
+        for (int i = 0; i < slices; ++i) {
+            const float* ml = slc.ml + ((int64_t)i * slc.rows + row) * 2;
+            const float m1 = ml[0], l1 = ml[1], mn = fmaxf(m, m1);
+            l = (m == -INFINITY ? 0.0f : l * exp2_small(m - mn)) +
+                (m1 == -INFINITY ? 0.0f : l1 * exp2_small(m1 - mn));
             m = mn;
         }
     }
-    {
-        const float m2 = __shfl_xor(m, 32, WAVE), l2 = __shfl_xor(l, 32, WAVE);
-        const float mn = fmaxf(m, m2);
-        l = (m == -INFINITY ? 0.0f : l * exp2_small((m - mn) * LOG2E)) +
-            (m2 == -INFINITY ? 0.0f : l2 * exp2_small((m2 - mn) * LOG2E));
-        m = mn;
-    }
-    if (h == 0) {
-        xch[qh][kh][c][0] = m;
-        xch[qh][kh][c][1] = l;
-    }
-    __syncthreads();
-    {
-        const float m0 = xch[qh][0][c][0], l0 = xch[qh][0][c][1];
-        const float m1 = xch[qh][1][c][0], l1 = xch[qh][1][c][1];
-        const float mn = fmaxf(m0, m1);
-        l = (m0 == -INFINITY ? 0.0f : l0 * exp2_small((m0 - mn) * LOG2E)) +
-            (m1 == -INFINITY ? 0.0f : l1 * exp2_small((m1 - mn) * LOG2E));
-        m = mn;
-    }
-    const float Lq = m + logf(l);
-    if (kh == 0 && h == 0) {
-        lse_out[head * T + q] = Lq;
-        d_out[head * T + q] = Dq;
-    }
+    if constexpr (PASS == LSE) return;
+    const float Lq = m + log2f(l);
+    if (kh == 0 && h == 0 && (int)blockIdx.y == 0) lse_out[row] = Lq;
 
     // Pass 2: dQ^T (rows d, columns queries) += K^T dS^T over the wave's keys.
     f32x16 dq0 = zero16(), dq1 = zero16();
-    for (int kb = 0; kb < nkb; ++kb) {
+    for (int kb = kb0; kb < nkb; ++kb) {
         block_load(Kh, kb * BT, rs, tid, kc);
         block_load(Vh, kb * BT, rs, tid, vc);
         __syncthreads();
@@ -279,11 +325,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const f32x16 pa = p2[0] + p2[1];
         float ds[16];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int key = kb * BT + 32 * kh + crow(v, h);
-            const float p = (causal && key > q) ? 0.0f : exp2_small((sa[v] * scale - Lq) * LOG2E);
-            ds[v] = p * (pa[v] - Dq);
+        for (int v = 0; v < 16; ++v) ds[v] = __builtin_fmaf(sa[v], sl, -Lq);
+        if (causal && kb == qb) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) ds[v] = 32 * kh + crow(v, h) > 32 * qh + c ? -INFINITY : ds[v];
         }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) ds[v] = exp2_small(ds[v]) * (pa[v] - Dq);
         // Slot (s, h) is key 32 kh + crow(s, h): this lane's ds[s].
         float ka[16], kb2[16];
 #pragma unroll
@@ -311,7 +359,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     __syncthreads();
     if (kh == 0) {
-        float* out = dQ + hoff + (int64_t)q * rs;
+        // A slice's partial is stored unscaled, rows of DH floats.
+        float* out = PASS == DQ ? slc.part + ((int64_t)blockIdx.y * slc.rows + row) * DH : dQ + hoff + (int64_t)q * rs;
+        if constexpr (PASS == DQ) scale = 1.0f;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             f32x4 a, b;
@@ -332,12 +382,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 
 // ── dK, dV ─────────────────────────────────────────────────────────────────
 // S tile = Q K^T (rows queries, columns keys): the lane's column is key
-// j = kb*64 + 32 kh + c; L and D of its 16 query rows come from LDS.
+// j = kb*64 + 32 kh + c; L and D of its 16 query rows come from LDS. SLICED:
+// blockIdx.y takes ck of the query blocks and stores partial dK and dV.
+template <bool SLICED>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dkdv_kernel(const float* __restrict__ Q, const float* __restrict__ K,
                                                                  const float* __restrict__ V, const float* __restrict__ dO,
                                                                  const float* __restrict__ lse, const float* __restrict__ dd,
                                                                  float* __restrict__ dK, float* __restrict__ dV, int T,
-                                                                 float scale, int causal, int hg, int rs) {
+                                                                 float scale, int causal, int hg, int rs, Slices slc) {
     // Q and dO blocks; at the end the qh = 1 partials ([kh][dK 64 + dV 64][33]).
     constexpr int SMEM = 2 * BT * PITCH > 2 * 128 * 33 ? 2 * BT * PITCH : 2 * 128 * 33;
     __shared__ __align__(16) float smem[SMEM];
@@ -351,6 +403,13 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int nkb = T / BT;
     int head_i, kb;
     block_of((int)blockIdx.x, (int)(gridDim.x / nkb), nkb, false, &head_i, &kb);
+    int qb0 = causal ? kb : 0, nqb = T / BT;
+    if constexpr (SLICED) {
+        qb0 += (int)blockIdx.y * slc.ck;
+        if (qb0 >= nqb) return;
+        nqb = min(nqb, qb0 + slc.ck);
+    }
+    const float sl = scale * LOG2E;  // scores in log2 units
     const int64_t head = head_i;
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
     const int qh = wave & 1, kh = wave >> 1, c = lane & 31, h = lane >> 5;
@@ -364,7 +423,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     f32x16 dk0 = zero16(), dk1 = zero16(), dv0 = zero16(), dv1 = zero16();
     // Blocks staged without prefetch (two workgroups per CU, as in the dQ kernel).
     f32x4 qc[4], oc[4];
-    const int qb0 = causal ? kb : 0, nqb = T / BT;
     const int lrow = tid < BT ? tid : 0, lslot = tid < BT ? tid : BT;
     const float* lse_h = lse + head * T;  // the head's L and D (uniform bases)
     const float* dd_h = dd + head * T;
@@ -405,11 +463,15 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const f32x16 pa = p2[0] + p2[1];
         float p[16], ds[16];
 #pragma unroll
+        for (int v = 0; v < 16; ++v) p[v] = __builtin_fmaf(sa[v], sl, -Ls[32 * qh + crow(v, h)]);
+        if (causal && kb == qb) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) p[v] = 32 * kh + c > 32 * qh + crow(v, h) ? -INFINITY : p[v];
+        }
+#pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int qi = 32 * qh + crow(v, h);
-            const bool masked = causal && j > qb * BT + qi;
-            p[v] = masked ? 0.0f : exp2_small((sa[v] * scale - Ls[qi]) * LOG2E);
-            ds[v] = p[v] * (pa[v] - Ds[qi]);
+            p[v] = exp2_small(p[v]);
+            ds[v] = p[v] * (pa[v] - Ds[32 * qh + crow(v, h)]);
         }
         // dV^T (rows d, columns keys) += dO^T P, dK^T += Q^T dS; slot (s, h)
         // is query 32 qh + crow(s, h): this lane's p[s] and ds[s].
@@ -452,6 +514,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
     if (qh == 0) {
         float* ok = dK + hoff + (int64_t)j * rs;
         float* ov = dV + hoff + (int64_t)j * rs;
+        if constexpr (SLICED) {
+            ok = slc.part + ((int64_t)(slc.n + blockIdx.y) * slc.rows + head * T + j) * DH;
+            ov = slc.part + ((int64_t)(2 * slc.n + blockIdx.y) * slc.rows + head * T + j) * DH;
+            scale = 1.0f;
+        }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const int d0 = 8 * g + 4 * h;
@@ -478,6 +545,23 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
             *reinterpret_cast<f32x4*>(ov + 32 + d0) = f;
         }
     }
+}
+
+// dQ, dK or dV (blockIdx.y) = the slices' partials in slice order, 4 floats a thread.
+__global__ __launch_bounds__(THREADS) void attn_bwd_sum_kernel(Slices p, float* __restrict__ dQ, float* __restrict__ dK,
+                                                               float* __restrict__ dV, int T, float scale, int causal,
+                                                               int hg, int rs) {
+    const int64_t e = ((int64_t)blockIdx.x * THREADS + threadIdx.x) * 4;
+    const int64_t row = e / DH, head = row / T;
+    if (row >= p.rows) return;
+    const int which = blockIdx.y, t = (int)(row - head * T), d = (int)(e % DH), nb = T / BT, blk = t / BT;
+    const int blocks = !causal ? nb : which == 0 ? blk + 1 : nb - blk;
+    const int n = (blocks + p.ck - 1) / p.ck;
+    const float* src = p.part + ((int64_t)which * p.n * p.rows + row) * DH + d;
+    f32x4 s = *reinterpret_cast<const f32x4*>(src);
+    for (int i = 1; i < n; ++i) s += *reinterpret_cast<const f32x4*>(src + (int64_t)i * p.rows * DH);
+    float* out = (which == 0 ? dQ : which == 1 ? dK : dV) + head_offset(head, T, hg, rs) + (int64_t)t * rs + d;
+    *reinterpret_cast<f32x4*>(out) = which == 2 ? s : s * scale;
 }
 
 }  // namespace
@@ -507,17 +591,55 @@ int attention_vjp(const float* q, const float* k, const float* v, const float* o
     const int64_t blocks = batch * (t / BT);
     if (blocks > int64_t(UINT32_MAX) / THREADS)
         return fail(MLXHIP_ERR_INVALID_ARGUMENT, "attention vjp: %lld heads exceed one launch", (long long)batch);
-    // L and D of every query row: [batch][t] each, in the stream's workspace.
+    // A workgroup's walk over all nb blocks of a sum takes about nb x 10 us on
+    // its CU. Where that is well over the whole work's share of a CU (units /
+    // 256), the blocks are sliced over workgroups, about two rounds of slices
+    // to a CU, and the partials added by one more launch. The launches and the
+    // partials cost about 3 blocks' time. Measured (dQ, dK and dV, us, causal
+    // unless noted, whole -> sliced): 1 head x 512 94 -> 30, 4 x 512 96 -> 33,
+    // 7 x 448 85 -> 49, 12 x 1024 191 -> 104, 4 x 2048 not causal 363 -> 171;
+    // but 64 x 192 46 against 54, 64 x 128 34 against 35.
+    const int nb = (int)(t / BT);
+    const int64_t rows = batch * t, units = batch * (causal ? (int64_t)nb * (nb + 1) / 2 : (int64_t)nb * nb);
+    Slices sl{};
+    if (units <= CUS * (nb - 3)) {
+        sl.ck = (int)ceil_div(units, 2 * CUS);
+        sl.n = (int)ceil_div(nb, sl.ck);
+        sl.rows = rows;
+    }
+    // L and D of every query row: [batch][t] each, in the stream's workspace,
+    // then the slices' pairs and partials; without room for those, unsliced.
     void* ws = nullptr;
-    MLXHIP_TRY(stream_workspace(s, WS_ATTN, (size_t)(2 * batch * t) * sizeof(float), &ws));
+    const size_t base = (size_t)(2 * rows) * sizeof(float);
+    if (sl.n > 1 && stream_workspace(s, WS_ATTN, base + (size_t)(sl.n * rows * (2 + 3 * DH)) * sizeof(float), &ws) != MLXHIP_OK)
+        sl.n = 0;
+    if (sl.n <= 1) MLXHIP_TRY(stream_workspace(s, WS_ATTN, base, &ws));
     float* lse = static_cast<float*>(ws);
-    float* dd = lse + batch * t;
-    hipLaunchKernelGGL(attn_bwd_dq_kernel, dim3((unsigned)blocks), dim3(THREADS), 0, s, q, k, v, o, dout, dq, lse, dd,
-                       (int)t, scale, causal, (int)hg, (int)rs);
+    float* dd = lse + rows;
+    const dim3 block(THREADS);
+    if (sl.n <= 1) {
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<WHOLE>), dim3((unsigned)blocks), block, 0, s, q, k, v, o, dout, dq, lse, dd,
+                           (int)t, scale, causal, (int)hg, (int)rs, sl);
+        MLXHIP_TRY(launch_check("attn_bwd_dq_kernel"));
+        hipLaunchKernelGGL((attn_bwd_dkdv_kernel<false>), dim3((unsigned)blocks), block, 0, s, q, k, v, dout, lse, dd, dk,
+                           dv, (int)t, scale, causal, (int)hg, (int)rs, sl);
+        return launch_check("attn_bwd_dkdv_kernel");
+    }
+    sl.part = dd + rows;  // 16-byte aligned: rows is a multiple of 64
+    sl.ml = sl.part + (int64_t)3 * sl.n * rows * DH;
+    const dim3 grid((unsigned)blocks, (unsigned)sl.n);
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<LSE>), grid, block, 0, s, q, k, v, o, dout, dq, lse, dd, (int)t, scale, causal,
+                       (int)hg, (int)rs, sl);
     MLXHIP_TRY(launch_check("attn_bwd_dq_kernel"));
-    hipLaunchKernelGGL(attn_bwd_dkdv_kernel, dim3((unsigned)blocks), dim3(THREADS), 0, s, q, k, v, dout, lse, dd, dk,
-                       dv, (int)t, scale, causal, (int)hg, (int)rs);
-    return launch_check("attn_bwd_dkdv_kernel");
+    hipLaunchKernelGGL((attn_bwd_dq_kernel<DQ>), grid, block, 0, s, q, k, v, o, dout, dq, lse, dd, (int)t, scale, causal,
+                       (int)hg, (int)rs, sl);
+    MLXHIP_TRY(launch_check("attn_bwd_dq_kernel"));
+    hipLaunchKernelGGL((attn_bwd_dkdv_kernel<true>), grid, block, 0, s, q, k, v, dout, lse, dd, dk, dv, (int)t, scale,
+                       causal, (int)hg, (int)rs, sl);
+    MLXHIP_TRY(launch_check("attn_bwd_dkdv_kernel"));
+    hipLaunchKernelGGL(attn_bwd_sum_kernel, dim3((unsigned)ceil_div(rows * DH / 4, THREADS), 3), block, 0, s, sl, dq, dk, dv,
+                       (int)t, scale, causal, (int)hg, (int)rs);
+    return launch_check("attn_bwd_sum_kernel");
 }
 
 }  // namespace mlxhip
