@@ -169,16 +169,31 @@ struct PackPair {
 };
 
 // One 16-byte chunk of a destination row: columns c0 .. c0 + CH - 1 of
-// source row r, zero outside rows x cols. Every element is loaded, from a
-// row and column clamped into range, before any is selected: a guarded load
-// per element compiles to a branch that waits for its own load.
+// source row r, zero outside rows x cols. Away from the row's end: one 16-byte
+// load from the dword at or below the first element (and for 16 bits the fifth
+// dword, and a shift by one element where that one is odd); every dword read
+// holds an element of the row. At the end every element is loaded, from a row
+// and column clamped into range, before any is selected: a guarded load per
+// element compiles to a branch that waits for its own load. With
+// element loads alone a packed product took longer by that much (bf16, us):
+// 2047 x 2047 x 2047 42.2 -> 38.6, 4095 x 1001 x 3001 55.4 -> 48.3.
 template <typename T, int CH>
 __device__ inline uint4 pack_chunk(const T* sb, int64_t ld, int64_t rows, int64_t cols, int64_t r, int64_t c0) {
+    typedef uint32_t dwords __attribute__((ext_vector_type(4), aligned(4)));
     union {
         uint4 v;
         T e[CH];
     } u;
     const T* src = sb + (r < rows ? r : rows - 1) * ld;
+    if (r < rows && c0 + CH < cols) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(src + c0);
+        const uint32_t* d = reinterpret_cast<const uint32_t*>(at & ~uintptr_t(3));
+        const dwords w = *reinterpret_cast<const dwords*>(d);
+        if constexpr (sizeof(T) == 4) return make_uint4(w.x, w.y, w.z, w.w);
+        const uint32_t w4 = d[4], sh = (uint32_t)(at & 2) * 8;
+        return make_uint4(__builtin_amdgcn_alignbit(w.y, w.x, sh), __builtin_amdgcn_alignbit(w.z, w.y, sh),
+                          __builtin_amdgcn_alignbit(w.w, w.z, sh), __builtin_amdgcn_alignbit(w4, w.w, sh));
+    }
     T t[CH];
 #pragma unroll
     for (int e = 0; e < CH; ++e) t[e] = src[c0 + e < cols ? c0 + e : cols - 1];
@@ -190,8 +205,7 @@ __device__ inline uint4 pack_chunk(const T* sb, int64_t ld, int64_t rows, int64_
 // Both operands of one GEMM in one launch (blockIdx.z picks the operand,
 // blockIdx.y the batch slice). Each thread writes one 16-byte chunk of a
 // destination row (cols_p is a multiple of the chunk and the destination is
-// 16-byte aligned); the source, whose rows need not be aligned, is read
-// element by element. An empty source (no rows or no columns) packs zeros.
+// 16-byte aligned); the source's rows need only element alignment. An empty source (no rows or no columns) packs zeros.
 template <typename T>
 __global__ __launch_bounds__(256) void pack_kernel(PackPair pp) {
     constexpr int CH = 16 / sizeof(T);
@@ -802,37 +816,51 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
                          ldc, stride_c, bias, aligned, s);
     }
     const int path = gemm_path();
+    // Zero-padded copies of both operands, whose rows are whole 16-byte chunks
+    // (K and the contiguous extents rounded up to a multiple of 16 bytes); the
+    // zero padding adds nothing to C. One stream-ordered allocation holds both
+    // (B at a 256-byte boundary) and one launch fills both: the host work per
+    // call is what small products wait on.
+    const int64_t kp = ceil_div(k, ch) * ch;
+    const int64_t a_rows = trans_a ? k : m;
+    const int64_t a_rows_p = trans_a ? kp : m, a_cols_p = ceil_div(a_cols, ch) * ch;
+    const int64_t b_rows = trans_b ? n : k;
+    const int64_t b_rows_p = trans_b ? n : kp, b_cols_p = ceil_div(b_cols, ch) * ch;
+    const size_t b_off = ((size_t)(a_rows_p * a_cols_p * batch * elem_size(ab_dtype)) + 255) & ~size_t(255);
+    const size_t pack_bytes = b_off + (size_t)(b_rows_p * b_cols_p * batch * elem_size(ab_dtype));
+    void* pa = nullptr;
+
     // 16-bit products the direct-to-LDS kernel cannot read as they are
     // (rows that are not whole 16-byte chunks) or that have too few 128 x 128
     // tiles to fill the chip: one launch of 64 x 64 tiles, no packed copies,
     // no K split. The odd 1000 x 777 x 1531 bf16 product: pack + split GEMM +
     // partial sums took ~25 us per call (three launches).
+    // Unaligned products of more tiles are packed: the 64 x 64 kernel runs one
+    // workgroup per CU, so every 256 tiles cost a round, at a quarter of the
+    // other kernel's rate. Measured (us, 64 x 64 / packed 128 x 128, NN bf16):
+    // 1409 x 1409 x 333 22.1 / 15.5, 1500 x 1501 x 777 36 / 22.5, 2000 x 1999 x
+    // 255 33 / 18.1, 2047 x 2047 x 2047 80 / 38.6, 2600 x 2601 x 4001 235 / 109,
+    // 4095 x 1001 x 3001 104 / 48, 1000 x 777 x 1531 in 4 slices 53 / 33. The
+    // line: half a round of 128 x 128 tiles, few of them mostly padding (300 x
+    // 301 x 2001 in 16 slices, 400 and 144 tiles: 36 / 45), and enough rows and
+    // columns to pay for the copies (121 x 16377 x 513: 24.4 / 24.6, NT 23.4 /
+    // 27.0). Only for a 16-bit C: the longer sums of one wave show in an f32
+    // one. Without room for the copies the product runs unpacked.
     if (ab_dtype != MLXHIP_DTYPE_F32 && (path == 6 || path == 0) && !padded &&
         gemm16_small_fits(m, n, k, batch, lda, ldb, trans_a, trans_b)) {
         const int64_t big_tiles = ceil_div(m, 256) * ceil_div(n, 256) * batch;
         const int64_t mid_tiles = ceil_div(m, 128) * ceil_div(n, 128) * batch;
+        const int64_t small_tiles = ceil_div(m, 64) * ceil_div(n, 64) * batch;
+        const bool pack = path == 0 && !aligned && c_dtype != MLXHIP_DTYPE_F32 && mid_tiles >= 128 && std::min(m, n) > 256 &&
+                          2 * small_tiles >= 7 * mid_tiles && pack_bytes <= (size_t(256) << 20) &&
+                          (!fs || pack_bytes <= fs->cap - std::min(fs->cap, fs->used + 255));
         if (path == 6 || (big_tiles < 128 && (!aligned || mid_tiles < 16)))
-            return gemm16_small(ab_dtype, c_dtype, trans_a, trans_b, m, n, k, batch, a, lda, stride_a, b, ldb,
-                                stride_b, c, ldc, stride_c, s);
+            if (!pack || take_workspace(fs, s, WS_PACK, pack_bytes, &pa) != MLXHIP_OK)
+                return gemm16_small(ab_dtype, c_dtype, trans_a, trans_b, m, n, k, batch, a, lda, stride_a, b, ldb,
+                                    stride_b, c, ldc, stride_c, s);
     }
     if (!aligned && path != 1) {
-        // Unaligned operands (odd leading dimension, offset pointer): copy both
-        // into zero-padded buffers whose rows are whole 16-byte chunks (K and
-        // the contiguous extents rounded up to a multiple of 16 bytes) and run
-        // the aligned kernels on those. The zero padding adds nothing to C.
-        const int64_t kp = ceil_div(k, ch) * ch;
-        const int64_t a_rows = trans_a ? k : m, a_cols = trans_a ? m : k;
-        const int64_t a_rows_p = trans_a ? kp : m, a_cols_p = ceil_div(a_cols, ch) * ch;
-        const int64_t b_rows = trans_b ? n : k, b_cols = trans_b ? k : n;
-        const int64_t b_rows_p = trans_b ? n : kp, b_cols_p = ceil_div(b_cols, ch) * ch;
-        const int es = elem_size(ab_dtype);
-        // One stream-ordered allocation holds both copies (B at a 256-byte
-        // boundary) and one launch fills both: the host work per call is
-        // what such small products wait on.
-        const size_t a_sz = (size_t)(a_rows_p * a_cols_p * batch * es);
-        const size_t b_off = (a_sz + 255) & ~size_t(255);
-        void* pa = nullptr;
-        MLXHIP_TRY(take_workspace(fs, s, WS_PACK, b_off + (size_t)(b_rows_p * b_cols_p * batch * es), &pa));
+        if (!pa) MLXHIP_TRY(take_workspace(fs, s, WS_PACK, pack_bytes, &pa));
         void* pb = static_cast<char*>(pa) + b_off;
         PackPair pp{{PackOp{a, lda, stride_a, a_rows, a_cols, pa, a_rows_p, a_cols_p},
                      PackOp{b, ldb, stride_b, b_rows, b_cols, pb, b_rows_p, b_cols_p}}};
@@ -888,7 +916,9 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
             // keeping at least 256 k (8 K tiles) per split. The 1000 x 777 x
             // 1531 product (56 tiles) runs 4 splits of 384 k on 224 CUs.
             int sp = 1;
-            if (cfg == 1 && path == 0)
+            // Packed operands: from 128 tiles on one workgroup per tile is faster (144
+            // tiles, K = 777: 24 us against 29 in two splits) and needs no partials.
+            if (cfg == 1 && path == 0 && !(padded && mid_tiles >= 128))
                 while (sp < 8 && mid_tiles * sp < 256 && k / (2 * sp) >= 256) sp *= 2;
             // MLXHIP_GEMM16_SPLITS=s forces the split factor (1..8; tuning).
             if (const char* e = getenv("MLXHIP_GEMM16_SPLITS")) {
