@@ -343,7 +343,10 @@ __device__ inline float fold(float v, float x) {
     return KIND == 2 ? fmaxf(v, x) : v + x;
 }
 
-template <int KIND>
+// SHORT: an axis of fewer than RED_SHORT elements, without the batches.
+constexpr int RED_SHORT = 8;
+
+template <int KIND, bool SHORT>
 __global__ __launch_bounds__(RED_BLOCK) void reduce_axis_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                                 int64_t outer, int64_t dim, int64_t inner) {
     for (int64_t f = (int64_t)blockIdx.x * RED_BLOCK + threadIdx.x; f < outer * inner;
@@ -351,6 +354,12 @@ __global__ __launch_bounds__(RED_BLOCK) void reduce_axis_kernel(const float* __r
         const int64_t o = f / inner, i = f % inner;
         const float* p = x + o * dim * inner + i;
         float v = KIND == 2 ? -INFINITY : -0.0f;
+        if constexpr (SHORT) {
+            for (int64_t d = 0; d < dim; ++d) v = fold<KIND>(v, p[d * inner]);
+            if (KIND == 1) v = v / (float)dim;
+            y[f] = v;
+            continue;
+        }
         // Two register batches in turn: batch b is loaded while batch a is
         // folded and the other way round, so memory latency overlaps the chain
         // of dependent adds; neither batch is ever copied (a copy would wait for
@@ -373,7 +382,30 @@ __global__ __launch_bounds__(RED_BLOCK) void reduce_axis_kernel(const float* __r
 #pragma unroll
             for (int u = 0; u < RED_U; ++u) v = fold<KIND>(v, b[u]);
         }
-        for (int64_t d = full; d < dim; ++d) v = fold<KIND>(v, p[d * inner]);
+        // The rest in batches of 64, 16 and 4, and the last ones together (past
+        // the end the last element is loaded again): a few at a time each cost
+        // a memory latency. us: [123, 4893] 14.0 -> 4.2, [511, 41] 18.4 -> 8.5,
+        // [100, 65537] 35.9 -> 8.7.
+        int64_t d = full;
+        auto batch = [&](auto U) {
+            for (; dim - d >= U; d += U) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) a[u] = p[(d + u) * inner];
+#pragma unroll
+                for (int u = 0; u < U; ++u) v = fold<KIND>(v, a[u]);
+            }
+        };
+        batch(std::integral_constant<int, RED_U>{});
+        batch(std::integral_constant<int, 16>{});
+        batch(std::integral_constant<int, 4>{});
+        if (d < dim) {
+            const int left = (int)(dim - d);
+#pragma unroll
+            for (int u = 0; u < 3; ++u) a[u] = p[(d + std::min(u, left - 1)) * inner];
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (u < left) v = fold<KIND>(v, a[u]);
+        }
         if (KIND == 1) v = v / (float)dim;
         y[f] = v;
     }
@@ -385,32 +417,41 @@ __global__ __launch_bounds__(RED_BLOCK) void reduce_axis_kernel(const float* __r
 // columns at the rate one CU can keep cache lines in flight. Here a
 // workgroup owns COLS outputs of one outer index: its 256 threads copy
 // chunks of RC_CH rows x COLS columns straight from memory into a ring of
-// LDS slots (buffer loads with the LDS flag, 16 bytes per lane, RC_P chunks
+// LDS slots (buffer loads with the LDS flag, VEC floats per lane, RC_P chunks
 // ahead), and COLS lanes of wave 0 fold each chunk in row order while the
 // next ones arrive. Rows past the end read as zero (out of the buffer's
 // range) and are never folded; columns past the end are never stored.
-// Needs inner % 4 == 0, a 16-byte aligned x and a slab of under 2^32 bytes.
+// Needs a slab of under 2^32 bytes, for VEC 4 also inner % 4 == 0 and a
+// 16-byte aligned x. VEC 1 takes every other row length and address: one
+// thread per output waited for each batch of 64 loads there ([3584, 41] 43.4
+// us, now 19.3; [2048, 1023] 26.3 -> 12.9; [14000, 1001] 173 -> 72).
 constexpr int RC_BLOCK = 256;
 
 #define MLXHIP_LDS_AS __attribute__((address_space(3)))
 
-// 16 bytes per lane from buffer offset `voff` into LDS at dst + 16 * lane.
+// VEC floats per lane from buffer offset `voff` into LDS at dst + 4 VEC * lane.
 // Inline assembly, so the compiler does not wait for these loads before
 // every LDS read; the kernel waits for them itself (vmcnt, then a barrier).
-__device__ inline void rc_lds_load16(__amdgpu_buffer_rsrc_t rsrc, MLXHIP_LDS_AS char* dst, uint32_t voff) {
+template <int VEC>
+__device__ inline void rc_lds_load(__amdgpu_buffer_rsrc_t rsrc, MLXHIP_LDS_AS char* dst, uint32_t voff) {
     const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)dst);
-    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
+    if constexpr (VEC == 4)
+        asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
+    else
+        asm volatile("buffer_load_dword %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc), "{m0}"(m0) : "memory");
 }
 
-template <int KIND, int COLS, int RC_CH, int RC_P, int FB>
+template <int KIND, int VEC, int COLS, int RC_CH, int RC_P, int FB>
 __global__ __launch_bounds__(RC_BLOCK) void reduce_cols_kernel(const float* __restrict__ x, float* __restrict__ y,
                                                                int64_t dim, int64_t inner, int64_t col_blocks) {
-    constexpr int TPR = COLS / 4;                       // lanes per row
-    constexpr int RPI = 64 / TPR;                       // rows per wave instruction (1 KiB)
+    constexpr int TPR = COLS / VEC;                     // lanes per row
+    constexpr int RPI = 64 / TPR;                       // rows per wave instruction
+    constexpr int WB = 64 * VEC * 4;                    // bytes per wave instruction
     constexpr int RC_NB = RC_P + 1;
     constexpr int CHUNK_BYTES = RC_CH * COLS * 4;
-    constexpr int L = CHUNK_BYTES / (RC_BLOCK * 16);    // loads per thread per chunk
-    static_assert(L * RC_BLOCK * 16 == CHUNK_BYTES, "whole 1 KiB blocks per wave");
+    constexpr int L = CHUNK_BYTES / (RC_BLOCK * VEC * 4);  // loads per thread per chunk
+    static_assert(L * RC_BLOCK * VEC * 4 == CHUNK_BYTES, "whole wave instructions");
+    static_assert(L * RC_P <= 63, "vmcnt counts the loads in flight");
     // The ring; the vmcnt below assumes these loads are the only vector
     // memory operations in flight.
     __shared__ __align__(16) float ring[RC_NB][RC_CH * COLS];
@@ -421,20 +462,20 @@ __global__ __launch_bounds__(RC_BLOCK) void reduce_cols_kernel(const float* __re
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)slab, (short)0, (int)(uint32_t)(dim * inner * 4), 0x00020000);
     // Load l of a chunk: wave instruction q = l * 4 + wave covers rows
-    // q * RPI .. q * RPI + RPI - 1 of the chunk; the lane's 16 bytes are
-    // row lane / TPR, columns c0 + 4 * (lane % TPR) .. + 3.
+    // q * RPI .. q * RPI + RPI - 1 of the chunk; the lane's VEC
+    // floats are row lane / TPR, columns c0 + VEC * (lane % TPR) and on.
     uint32_t voff[L];
 #pragma unroll
     for (int l = 0; l < L; ++l) {
         const int64_t row = (int64_t)(l * 4 + wave) * RPI + lane / TPR;
-        voff[l] = (uint32_t)((row * inner + c0 + 4 * (lane % TPR)) * 4);
+        voff[l] = (uint32_t)((row * inner + c0 + VEC * (lane % TPR)) * 4);
     }
     const uint32_t chunk_step = (uint32_t)(RC_CH * inner * 4);
     auto issue = [&](int ch) {
         MLXHIP_LDS_AS char* slot = (MLXHIP_LDS_AS char*)&ring[ch % RC_NB][0];
 #pragma unroll
         for (int l = 0; l < L; ++l)
-            rc_lds_load16(rsrc, slot + (l * 4 + wave) * 1024, voff[l] + (uint32_t)ch * chunk_step);
+            rc_lds_load<VEC>(rsrc, slot + (l * 4 + wave) * WB, voff[l] + (uint32_t)ch * chunk_step);
     };
     const int nch = (int)((dim + RC_CH - 1) / RC_CH);
     float v = KIND == 2 ? -INFINITY : -0.0f;
@@ -973,6 +1014,21 @@ int reduce_rows(int kind, const float* x, float* y, int64_t rows, int64_t dim, h
     return vec ? launch_reduce_rows<4, 4>(kind, x, y, rows, dim, s) : launch_reduce_rows<4, 1>(kind, x, y, rows, dim, s);
 }
 
+constexpr int RC_COLS = 16, RC_CH_ROWS = 256, RC_AHEAD = 4, RC_FB = 32;
+
+template <int VEC, int P>
+int launch_reduce_cols(int kind, const float* x, float* y, int64_t outer, int64_t dim, int64_t inner, hipStream_t s) {
+    const int64_t cb = ceil_div(inner, RC_COLS);
+    const dim3 g((unsigned)(outer * cb)), b(RC_BLOCK);
+    if (kind == 0)
+        hipLaunchKernelGGL((reduce_cols_kernel<0, VEC, RC_COLS, RC_CH_ROWS, P, RC_FB>), g, b, 0, s, x, y, dim, inner, cb);
+    else if (kind == 1)
+        hipLaunchKernelGGL((reduce_cols_kernel<1, VEC, RC_COLS, RC_CH_ROWS, P, RC_FB>), g, b, 0, s, x, y, dim, inner, cb);
+    else
+        hipLaunchKernelGGL((reduce_cols_kernel<2, VEC, RC_COLS, RC_CH_ROWS, P, RC_FB>), g, b, 0, s, x, y, dim, inner, cb);
+    return launch_check("reduce_cols_kernel");
+}
+
 }  // namespace
 
 int reduce_axis(int kind, const float* x, float* y, int64_t outer, int64_t dim, int64_t inner,
@@ -982,29 +1038,32 @@ int reduce_axis(int kind, const float* x, float* y, int64_t outer, int64_t dim, 
     // Contiguous rows; below 64 elements a row is a line or two, and one thread
     // per row reads it as fast ([16384, 63] 12 us either way).
     if (inner == 1 && dim >= 64 && ceil_div(outer, 4) < (int64_t(1) << 23)) return reduce_rows(kind, x, y, outer, dim, s);
-    // Long axes over float4-aligned rows: the chunked LDS fold (same order).
-    // Chunks of 256 rows, 4 in flight, folded from 32-row register batches:
-    // the fastest of the chunk / prefetch / batch sizes measured on Sum over
-    // 2048 rows of 1024 and 4096 columns (11.1 and 16.4 us, against 25.8 and
-    // 26.3 us for one thread per output). Offsets up to P + 1 chunks past
-    // the last row stay below 2^32.
-    constexpr int CH = 256, PF = 4, FB = 32, COLS = 16;
-    if (dim >= 2 * CH && inner % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-        (dim + (PF + 1) * CH) * inner * 4 < (int64_t(1) << 32) && outer * ceil_div(inner, COLS) < (int64_t(1) << 31)) {
-        const int64_t cb = ceil_div(inner, COLS);
-        const dim3 g((unsigned)(outer * cb));
-        if (kind == 0)
-            hipLaunchKernelGGL((reduce_cols_kernel<0, COLS, CH, PF, FB>), g, dim3(RC_BLOCK), 0, s, x, y, dim, inner, cb);
-        else if (kind == 1)
-            hipLaunchKernelGGL((reduce_cols_kernel<1, COLS, CH, PF, FB>), g, dim3(RC_BLOCK), 0, s, x, y, dim, inner, cb);
-        else
-            hipLaunchKernelGGL((reduce_cols_kernel<2, COLS, CH, PF, FB>), g, dim3(RC_BLOCK), 0, s, x, y, dim, inner, cb);
-        return launch_check("reduce_cols_kernel");
-    }
+    // Long axes: the chunked LDS fold (same order). Chunks of 256 rows, 4 in
+    // flight, folded from 32-row register batches: the fastest of the chunk /
+    // prefetch / batch sizes measured on Sum over 2048 rows of 1024 and 4096
+    // columns (11.1 and 16.4 us, against 25.8 and 26.3 us for one thread per
+    // output). Offsets up to P + 1 chunks past the last row stay below 2^32.
+    // Rows that are no whole 16 bytes take four times the loads (3 chunks in
+    // flight): that pays while the workgroups find a CU each (us, one thread per
+    // output / here: 2048 rows of 1023 26.3 / 12.9, 4095 26.3 / 18.6, 8191 27 /
+    // 32; 1024 rows of 16383 18 / 38).
+    const int64_t blocks = outer * ceil_div(inner, RC_COLS);
+    const bool vec = inner % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    if (dim >= 2 * RC_CH_ROWS && (dim + (RC_AHEAD + 1) * RC_CH_ROWS) * inner * 4 < (int64_t(1) << 32) &&
+        blocks < (vec ? int64_t(1) << 31 : 257))
+        return vec ? launch_reduce_cols<4, RC_AHEAD>(kind, x, y, outer, dim, inner, s)
+                   : launch_reduce_cols<1, RC_AHEAD - 1>(kind, x, y, outer, dim, inner, s);
     const dim3 grid((unsigned)std::min<int64_t>(ceil_div(n, RED_BLOCK), MAX_GRID));
-    if (kind == 0) hipLaunchKernelGGL(reduce_axis_kernel<0>, grid, dim3(RED_BLOCK), 0, s, x, y, outer, dim, inner);
-    else if (kind == 1) hipLaunchKernelGGL(reduce_axis_kernel<1>, grid, dim3(RED_BLOCK), 0, s, x, y, outer, dim, inner);
-    else hipLaunchKernelGGL(reduce_axis_kernel<2>, grid, dim3(RED_BLOCK), 0, s, x, y, outer, dim, inner);
+    const dim3 block(RED_BLOCK);
+    auto launch = [&](auto sh) {
+        constexpr bool SHORT = decltype(sh)::value;
+        if (kind == 0) hipLaunchKernelGGL((reduce_axis_kernel<0, SHORT>), grid, block, 0, s, x, y, outer, dim, inner);
+        else if (kind == 1) hipLaunchKernelGGL((reduce_axis_kernel<1, SHORT>), grid, block, 0, s, x, y, outer, dim, inner);
+        else hipLaunchKernelGGL((reduce_axis_kernel<2, SHORT>), grid, block, 0, s, x, y, outer, dim, inner);
+    };
+    // An axis of 3 over a million outputs: 16.6 us with the batches, 13.2 without.
+    if (dim < RED_SHORT) launch(std::true_type{});
+    else launch(std::false_type{});
     return launch_check("reduce_axis_kernel");
 }
 

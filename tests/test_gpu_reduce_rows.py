@@ -41,3 +41,24 @@ def test_whole_tensor_folds_in_order(n, kind):
     want = CpuRefBackend().eval_node(op, [NodeInput(x, x.shape)], meta([]))
     got = hb.HipBackend().eval_node(op, [NodeInput(x, x.shape)], meta([]))
     np.testing.assert_array_equal(got.view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("shape", [(2, 3), (1, 7), (1, 8), (1, 15), (1, 17), (2, 63), (1, 65), (1, 127), (1, 129), (3, 255), (1, 511),
+                                   (1, 512), (2, 513), (1, 1023), (1, 1025), (3, 1537)])
+@pytest.mark.parametrize("inner", [2, 15, 17, 63, 64, 65])
+@pytest.mark.parametrize("kind", ["sum", "mean", "max"])
+def test_columns_fold_in_order(shape, inner, kind):
+    """The middle axis at the edges of the register batches (16, 64, 128) and
+    of the LDS chunks (256 rows, 16 columns), rows at every alignment."""
+    op = {"sum": OpKind.Sum, "mean": OpKind.Mean, "max": OpKind.Max}[kind](1)
+    outer, dim = shape
+    x = np.random.default_rng(dim + inner).standard_normal((outer, dim, inner), dtype=np.float32) * 3 + 1
+    x[0, :, 0] = -0.0
+    x[0, dim - 1, 1] = -np.inf
+    want = CpuRefBackend().eval_node(op, [NodeInput(x.reshape(-1), x.shape)], meta([outer, inner]))
+    d = hb.DeviceBuffer(x.nbytes + 16)
+    d.upload(x, offset=4)
+    y = hb.DeviceBuffer(4 * outer * inner)
+    hb.eval_node_dev(op, [(d.ptr + 4, x.shape)], meta([outer, inner]), y)
+    hb.synchronize()
+    np.testing.assert_array_equal(y.download().view(np.uint32), np.asarray(want, np.float32).reshape(-1).view(np.uint32))
