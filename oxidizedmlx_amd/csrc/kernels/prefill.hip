@@ -310,7 +310,8 @@ __global__ __launch_bounds__(ATT_BLOCK) void prefill_attn_kernel(const float* __
     // The longest queries first: the last round is then the shortest.
     const int p0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * Q;
     const int nq = min(Q, cp - p0);
-    const int T = t0 + p0 + nq;  // positions the last query sees; query i sees T - nq + 1 + i
+    const int T = t0 + p0 + nq;       // positions the last query sees; query i sees T - nq + 1 + i
+    const int T0 = t0 + p0 + 1;       // and all of them see these
     int Ti[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) Ti[i] = t0 + p0 + min(i, nq - 1) + 1;
@@ -326,11 +327,17 @@ __global__ __launch_bounds__(ATT_BLOCK) void prefill_attn_kernel(const float* __
     auto load_v = [&](int j0) {
 #pragma unroll
         for (int u = 0; u < VCH; ++u) {
-            const int j = min(j0 + u * G, T - 1);
+            const int j = min(j0 + u * G, T0 - 1);
             vr[u] = *reinterpret_cast<const float4*>(vv + (int64_t)j * HD + 4 * c);
         }
     };
     load_v(g);
+    // A row past T0 is some of the queries' only: not 0 times a V that may have
+    // overflowed for the others. At most one of them is this thread's.
+    static_assert(Q - 1 <= G, "one row past T0 per position group");
+    const int jt = T0 + (g + G - T0 % G) % G;
+    float4 vt;
+    if constexpr (Q > 1) vt = *reinterpret_cast<const float4*>(vv + (int64_t)min(jt, T - 1) * HD + 4 * c);
     __syncthreads();  // the queries
 
     constexpr int KCH = HD < 32 ? HD : 32;
@@ -397,7 +404,7 @@ __global__ __launch_bounds__(ATT_BLOCK) void prefill_attn_kernel(const float* __
     float4 acc[Q];
 #pragma unroll
     for (int i = 0; i < Q; ++i) acc[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (int j0 = g; j0 < T; j0 += G * VCH) {
+    for (int j0 = g; j0 < T0; j0 += G * VCH) {
         if (j0 != g) load_v(j0);
 #pragma unroll
         for (int u = 0; u < VCH; ++u) {
@@ -405,12 +412,22 @@ __global__ __launch_bounds__(ATT_BLOCK) void prefill_attn_kernel(const float* __
 #pragma unroll
             for (int i = 0; i < Q; ++i) {
                 const float pj =
-                    j < Ti[i] ? s[i * sld + j] * pick4((j >> 6) & 3, f[i][0], f[i][1], f[i][2], f[i][3]) : 0.0f;
+                    j < T0 ? s[i * sld + j] * pick4((j >> 6) & 3, f[i][0], f[i][1], f[i][2], f[i][3]) : 0.0f;
                 acc[i].x += pj * vr[u].x;
                 acc[i].y += pj * vr[u].y;
                 acc[i].z += pj * vr[u].z;
                 acc[i].w += pj * vr[u].w;
             }
+        }
+    }
+#pragma unroll
+    for (int i = 1; i < Q; ++i) {
+        if (jt < Ti[i]) {
+            const float pj = s[i * sld + jt] * pick4((jt >> 6) & 3, f[i][0], f[i][1], f[i][2], f[i][3]);
+            acc[i].x += pj * vt.x;
+            acc[i].y += pj * vt.y;
+            acc[i].z += pj * vt.z;
+            acc[i].w += pj * vt.w;
         }
     }
 #pragma unroll

@@ -9,7 +9,7 @@ runs the same positions as a prompt."""
 import numpy as np
 import pytest
 
-from oxidizedmlx_amd import nn
+from oxidizedmlx_amd import abi, nn
 from oxidizedmlx_amd.backend import HipDecoder
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip")]
@@ -47,3 +47,48 @@ def test_prompt_positions_have_the_steps_bits(d, heads, ratio, vocab, layers, ba
         np.testing.assert_array_equal(dec.generate(seq[:, :-3], 4), am[:, -4:])
         np.testing.assert_array_equal(dec.generate(seq[:, :-3], 4, eager=True), am[:, -4:])
     dec.close()
+
+
+@pytest.mark.parametrize("d,heads,positions,hot", [
+    (64, 4, 11, 3), (64, 4, 11, 6), (64, 4, 11, 9),  # the last, third and second of four queries
+    (128, 2, 300, 290),                              # beyond the V rows that are loaded first
+    (256, 1, 70, 5),                                 # and with whole chunks of V rows behind it
+])
+def test_values_that_overflow_stay_with_the_positions_that_see_them(d, heads, positions, hot):
+    """A token whose V overflows in the first layer: positions before it have
+    the logits of a step per position (and of a prompt without that token),
+    positions from it on are NaN where the steps are. The steps: the same
+    prompt with no device memory for a pass of many positions."""
+    print(f"prefill overflow d={d} heads={heads} positions={positions} hot={hot}", flush=True)
+    vocab, batch = 64, 2
+    cfg = nn.DecoderConfig(n_layers=2, d_model=d, n_heads=heads, vocab=vocab, max_batch=batch, max_seq=positions + 1)
+    p = nn.decoder_params(cfg, d + hot)
+    p["embedding"][:, 0] = 0.0
+    p["embedding"][7] = 0.0
+    p["embedding"][7, 0] = 1.0
+    p["layers"][0]["wv"][:, 0] = 3e38  # x / rms is sqrt(d) in that column
+    dec = HipDecoder(cfg)
+    dec.load(p)
+    seq = np.random.default_rng(hot).integers(8, vocab, size=(batch, positions))
+    _, clean, lclean = dec.generate(seq, 1, argmax=True, logits=True)
+    assert np.isfinite(lclean).all()
+    seq[0, hot] = 7
+    _, am, lg = dec.generate(seq, 1, argmax=True, logits=True)
+    dec.close()
+    dec = HipDecoder(cfg)
+    dec.load(p)
+    dec.generate(seq[:, :2], positions - 1, logits=True)  # room for the logits
+    L = abi.load_library()
+    L.mlxhip_debug_fail_allocations(0)
+    try:
+        _, sam, slg = dec.generate(seq, 1, argmax=True, logits=True)
+    finally:
+        L.mlxhip_debug_fail_allocations(-1)
+    dec.close()
+    assert np.isnan(slg[0, hot:]).all()
+    np.testing.assert_array_equal(np.isnan(lg), np.isnan(slg))
+    for b, n in ((0, hot), (1, positions)):
+        np.testing.assert_array_equal(lg[b, :n].view(np.uint32), slg[b, :n].view(np.uint32))
+        np.testing.assert_array_equal(lg[b, :n].view(np.uint32), lclean[b, :n].view(np.uint32))
+        np.testing.assert_array_equal(am[b, :n], sam[b, :n])
+        np.testing.assert_array_equal(am[b, :n], clean[b, :n])
