@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -107,17 +108,10 @@ __device__ inline void row_reduce_max_sum(float& m, float& s, float* slot, int w
             slot[2 * wave_in_row + 1] = s;
         }
         __syncthreads();
-        if constexpr (WPR > 4) {
-            m = slot[2 * (lane % WPR)];
-            s = slot[2 * (lane % WPR) + 1];
+        m = slot[0];
+        s = slot[1];
 #pragma unroll
-            for (int o = WPR / 2; o > 0; o >>= 1) merge_max_sum(m, s, __shfl_xor(m, o, WAVE), __shfl_xor(s, o, WAVE));
-        } else {
-            m = slot[0];
-            s = slot[1];
-#pragma unroll
-            for (int w = 1; w < WPR; ++w) merge_max_sum(m, s, slot[2 * w], slot[2 * w + 1]);
-        }
+        for (int w = 1; w < WPR; ++w) merge_max_sum(m, s, slot[2 * w], slot[2 * w + 1]);
     }
 }
 
@@ -255,27 +249,34 @@ enum RowFill { FILL_EVEN = 0, FILL_VECS = 1, FILL_ANY = 2 };
 
 constexpr int VEC = 4;
 constexpr int row_block(int wpr) { return wpr > 4 ? wpr * WAVE : BLOCK; }
+constexpr bool row_softmax(int op) { return op == ROW_SOFTMAX || op == ROW_SCALED_MASKED_SOFTMAX; }
 constexpr bool row_two(int op) { return op == ROW_SOFTMAX_VJP || op == ROW_LAYERNORM_VJP || op == ROW_RMSNORM_VJP; }
 
-// exp(d) for d <= 0 to about an ulp: 2^(d log2 e) with the product's rounding
-// error (and that of the constant) carried to first order.
-__device__ inline float exp_small(float d) {
-    constexpr float L = 1.44269502162933349609375f, L_LO = 1.92596299112661746887e-8f, LN2 = 0.693147182464599609375f;
-    d = d < -200.0f ? -200.0f : d;  // 0 either way; keeps -inf out of the error term and NaN in
-    const float t = d * L;
-    const float e = __builtin_fmaf(d, L_LO, __builtin_fmaf(d, L, -t));
-    const float r = __builtin_amdgcn_exp2f(t);
-    return __builtin_fmaf(r, e * LN2, r);
+constexpr int row_waves_per_simd(int op, int wpr) {
+    return wpr == 16 && row_softmax(op) ? 8 : wpr > 4 ? wpr / 4 : row_two(op) ? 2 : 4;
+}
+
+// exp(x - m) for x <= m, as 2^n 2^f with d log2 e = n + f, d = x - m. The
+// rounding errors of d (lo: exact where |m| >= |x|, else to half a last place
+// of x) and of log2 e are added to f; only v_exp_f32's remains.
+__device__ inline float exp_below(float x, float m) {
+    constexpr float L = 1.44269502162933349609375f, L_LO = 1.92596299112661746887e-8f;
+    const float d = x - m, lo = x - (d + m);
+    const float n = __builtin_rintf(d * L);
+    const float f = __builtin_fmaf(lo, L, __builtin_fmaf(d, L_LO, __builtin_fmaf(d, L, -n)));
+    const float r = __builtin_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
+    return d < -200.0f ? 0.0f : r;  // -inf too; NaN stays
 }
 
 // a: x (forward) or dy (VJP); b: second operand of a VJP (softmax output s,
 // or the forward input x). p: eps or scale.
 // Single-input ops are held to 128 VGPRs so four 256-thread workgroups (16
 // waves) are resident per CU: a [4096, 4096] problem is 1024 workgroups, i.e.
-// exactly one round on 256 CUs.
+// exactly one round on 256 CUs. A softmax over 16 waves is held to 64, for two
+// workgroups per CU.
 template <int OP, int WPR, int NV, int FILL>
 __global__ __launch_bounds__(row_block(WPR)) __attribute__((amdgpu_waves_per_eu(
-    WPR > 4 ? WPR / 4 : row_two(OP) ? 2 : 4))) void row_kernel(const float* __restrict__ a,
+    row_waves_per_simd(OP, WPR)))) void row_kernel(const float* __restrict__ a,
                                                     const float* __restrict__ b,
                                                     float* __restrict__ y, int64_t rows,
                                                     int cols, float p, int causal) {
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(row_block(WPR)) __attribute__((amdgpu_waves_per_eu(
     auto has = [&](int j, int e) { return EVEN || (FILL == FILL_ANY ? e < have[j] : have[j] != 0); };
     const float d = (float)cols;
 
-    if constexpr (OP == ROW_SOFTMAX || OP == ROW_SCALED_MASKED_SOFTMAX) {
+    if constexpr (row_softmax(OP)) {
         if constexpr (OP == ROW_SCALED_MASKED_SOFTMAX) {
 #pragma unroll
             for (int j = 0; j < NV; ++j)
@@ -343,14 +344,6 @@ __global__ __launch_bounds__(row_block(WPR)) __attribute__((amdgpu_waves_per_eu(
                     v[j * VEC + e] = x;
                 }
         }
-        // Lane statistics (m, s = sum exp(x - m)) merged across the row in
-        // one exchange; then y = exp(x - m_row) / s_row, each lane's stored
-        // exp(x - m_lane) rescaled by exp(m_lane - m_row). exp(d) is
-        // 2^(d log2 e) on arguments d <= 0: relative error ~|d| * 2^-24 plus
-        // one v_exp_f32 ulp per factor, far inside the 1e-5 tolerance, at a
-        // quarter of expf's VALU cost. Rows of 16 waves carry the rounding
-        // errors along (exp_small): as exact as the expf that they had before.
-        constexpr bool LONG = WPR == 16;
         float ml = -INFINITY;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
@@ -361,29 +354,66 @@ __global__ __launch_bounds__(row_block(WPR)) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int e = 0; e < VEC; ++e) ml = fmaxf(ml, v[j * VEC + e]);
         }
-        // A lane whose values are all -inf adds nothing (its exps are 0
-        // against any finite row maximum); a row that is all -inf still ends
-        // as NaN, as exp(-inf - -inf) makes it in the reference.
-        const float mx = ml == -INFINITY ? 0.0f : ml;
-        float s = 0.0f;
+        float s = 0.0f, r;
+        if constexpr (WPR > 4) {
+            // exp(x - m_wave) before the exchange, which the other waves' loads
+            // hide (against m_row after it, [1048, 32003] took 57 us, not 53.5);
+            // after it one factor per wave, exp(m_wave - m_row) / s_row. In double
+            // for 16 waves, where that costs nothing; for 8 waves it cost 4 us of
+            // 50 ([5592, 6000]). Errors against float64, N(0, 2^2), root mean
+            // square over the values and relative in the 2-norm: 16 waves 4.6e-8
+            // and 3.5e-8, 8 waves 6.6e-8 and 5.7e-8; expf(x - m_row) / s, which
+            // ragged rows of this length had, 2.1-2.4e-7 and 6.0-6.3e-8.
+            const float mw = wave_max(ml), mx = mw == -INFINITY ? 0.0f : mw;  // all -inf: as below
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {
-                const float d = v[j * VEC + e] - mx;
-                const float ex = LONG ? exp_small(d) : __builtin_amdgcn_exp2f(d * 1.44269504088896340736f);
-                v[j * VEC + e] = ex;
-                s += ex;
+            for (int j = 0; j < N; ++j) {
+                v[j] = exp_below(v[j], mx);
+                s += v[j];
             }
-        float m = ml;
-        row_reduce_max_sum<WPR>(m, s, slot0, wave_in_row, lane);
-        const float scale = ml == -INFINITY ? 0.0f
-                            : LONG ? exp_small(ml - m)
-                                   : __builtin_amdgcn_exp2f((ml - m) * 1.44269504088896340736f);
-        float r;
-        row_divisor(s, r);
+            s = wave_sum(s);
+            if (lane == 0) {
+                slot0[2 * wave_in_row] = mw;
+                slot0[2 * wave_in_row + 1] = s;
+            }
+            __syncthreads();
+            // Lane i takes wave i % WPR's pair.
+            const float mi = slot0[2 * (lane % WPR)];
+            float m = mi;
 #pragma unroll
-        for (int j = 0; j < N; ++j) v[j] = div_by(v[j] * scale, s, r);
+            for (int o = WPR / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, WAVE));
+            using F = std::conditional_t<WPR == 16, double, float>;
+            F f;
+            if constexpr (WPR == 16) f = exp((double)mi - (double)m);
+            else f = exp_below(mi, m);
+            F sum = f * (F)slot0[2 * (lane % WPR) + 1];
+#pragma unroll
+            for (int o = WPR / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o, WAVE);
+            r = (float)(__shfl(f, wave_in_row, WAVE) / sum);
+#pragma unroll
+            for (int j = 0; j < N; ++j) v[j] *= r;
+        } else {
+            // Lane statistics (m, s = sum exp(x - m)) merged across the row in
+            // one exchange; then y = exp(x - m_row) / s_row, each lane's stored
+            // exp(x - m_lane) rescaled by exp(m_lane - m_row). exp(d) is
+            // 2^(d log2 e) on arguments d <= 0: relative error ~|d| * 2^-24 plus
+            // one v_exp_f32 ulp per factor, far inside the 1e-5 tolerance, at a
+            // quarter of expf's VALU cost.
+            // A lane whose values are all -inf adds nothing (its exps are 0
+            // against any finite row maximum); a row that is all -inf still ends
+            // as NaN, as exp(-inf - -inf) makes it in the reference.
+            const float mx = ml == -INFINITY ? 0.0f : ml;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                v[j] = __builtin_amdgcn_exp2f((v[j] - mx) * 1.44269504088896340736f);
+                s += v[j];
+            }
+            float m = ml;
+            row_reduce_max_sum<WPR>(m, s, slot0, wave_in_row, lane);
+            const float scale = ml == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ml - m) * 1.44269504088896340736f);
+            row_divisor(s, r);
+#pragma unroll
+            for (int j = 0; j < N; ++j) v[j] = div_by(v[j] * scale, s, r);
+        }
     } else if constexpr (OP == ROW_LAYERNORM) {
         // Lane moments (count, mean, sum of squared deviations) by an exact
         // two-pass over the lane's values, merged across the row in one

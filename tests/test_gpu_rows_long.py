@@ -53,3 +53,23 @@ def test_special_values_beside_partial_vectors(cols):
         want = oracle(OpKind.Softmax(-1), x)
     y = run_rows(hb.softmax_rows, x)
     np.testing.assert_allclose(y, want, rtol=1e-5, atol=1e-7, equal_nan=True)
+
+
+@pytest.mark.parametrize("cols,offset", [(4097, 0), (6000, 0), (6000, 1), (8190, 0), (8192, 0), (8195, 0), (12000, 0),
+                                         (16383, 0), (16384, 3), (20001, 0), (32003, 0), (32768, 0)])
+def test_softmax_of_long_rows_is_as_exact_as_expf(cols, offset):
+    """Each value's relative error against float64. exp(x - m) has one unit in
+    the last place of v_exp_f32 (2^-23) and, of the difference's rounding, at
+    most half a last place of x (|x| < 16: 2^-21); the wave's factor as much
+    again without the latter and a rounding, the product one: below 1e-6 in
+    all, and 1e-7 in the root mean square (about 3.4e-8 per rounding of 2^-24,
+    at most six of them). expf against the row's maximum, whose difference is
+    rounded, has 2.1e-7 to 2.4e-7."""
+    rows = (1 << 18) // cols
+    x = synth.normal(cols + offset, (rows, cols), 0.0, 2.0)
+    y = run_rows(hb.softmax_rows, x, offset=offset).astype(np.float64)
+    z = np.exp(x.astype(np.float64) - x.max(1, keepdims=True))
+    err = y / (z / z.sum(1, keepdims=True)) - 1
+    rms, worst = np.sqrt(np.square(err).mean()), np.abs(err).max()
+    print(f"softmax {rows}x{cols}+{offset}: rms {rms:.2e} max {worst:.2e}", flush=True)
+    assert rms <= 1e-7 and worst <= 1e-6
