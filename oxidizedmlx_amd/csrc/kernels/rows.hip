@@ -32,6 +32,7 @@
 #include "../common.hpp"
 #include "../kernels.hpp"
 #include "device_math.hpp"
+#include "row_launch.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -654,6 +655,7 @@ template <int OP, int WPR, int NV>
 int launch_rows(const float* a, const float* b, float* y, int64_t rows, int64_t cols, float p,
                 int causal, hipStream_t s) {
     constexpr int RPB = row_block(WPR) / (WAVE * WPR);
+    static_assert(WAVE * WPR <= row_threads(NV * VEC * WAVE * WPR), "row_chunk counts every work-item");
     const dim3 grid((unsigned)ceil_div(rows, RPB)), block(row_block(WPR));
     const uintptr_t at = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(y) |
                          (row_two(OP) ? reinterpret_cast<uintptr_t>(b) : 0);
@@ -714,34 +716,23 @@ int row_op(int op, const float* a, const float* b, float* y, int64_t rows, int64
     if (rows < 0 || cols < 0) return fail(MLXHIP_ERR_INVALID_ARGUMENT, "row op: negative size");
     if (rows > (int64_t)INT32_MAX) return fail(MLXHIP_ERR_INVALID_ARGUMENT, "row op: too many rows");
     if (cols > INT32_MAX) return fail(MLXHIP_ERR_INVALID_ARGUMENT, "row op: row too long");
-    // Rows are independent: a long non-causal batch runs as launches of at
-    // most ROW_CHUNK rows, so no grid (up to 256 work-items per row) exceeds
-    // the 32-bit work-item count of a dispatch. A causal mask is indexed by
-    // the row, and causal score matrices are far below that size.
-    constexpr int64_t ROW_CHUNK = int64_t(1) << 22;
-    if (rows > ROW_CHUNK && !causal) {
-        for (int64_t r0 = 0; r0 < rows; r0 += ROW_CHUNK) {
-            const int64_t off = r0 * cols, n = std::min(ROW_CHUNK, rows - r0);
-            MLXHIP_TRY(row_op(op, a + off, b ? b + off : nullptr, y + off, n, cols, p, 0, s));
-        }
-        return MLXHIP_OK;
-    }
     // MLXHIP_ROW_WPR forces the waves per row (tuning); 0 / unset = automatic.
     const int fw = row_force_wpr();
-    switch (op) {
-        case ROW_SOFTMAX: return dispatch_rows<ROW_SOFTMAX>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_SCALED_MASKED_SOFTMAX:
-            return dispatch_rows<ROW_SCALED_MASKED_SOFTMAX>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_LAYERNORM: return dispatch_rows<ROW_LAYERNORM>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_RMSNORM: return dispatch_rows<ROW_RMSNORM>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_SOFTMAX_VJP:
-            return dispatch_rows<ROW_SOFTMAX_VJP>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_LAYERNORM_VJP:
-            return dispatch_rows<ROW_LAYERNORM_VJP>(a, b, y, rows, cols, p, causal, s, fw);
-        case ROW_RMSNORM_VJP:
-            return dispatch_rows<ROW_RMSNORM_VJP>(a, b, y, rows, cols, p, causal, s, fw);
-        default: return fail(MLXHIP_ERR_INVALID_ARGUMENT, "row op: unknown op %d", op);
-    }
+    return for_row_chunks(rows, cols, causal, [&](int64_t r0, int64_t n, int mask) {
+        const float *ca = a + r0 * cols, *cb = b ? b + r0 * cols : nullptr;
+        float* cy = y + r0 * cols;
+        switch (op) {
+            case ROW_SOFTMAX: return dispatch_rows<ROW_SOFTMAX>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_SCALED_MASKED_SOFTMAX:
+                return dispatch_rows<ROW_SCALED_MASKED_SOFTMAX>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_LAYERNORM: return dispatch_rows<ROW_LAYERNORM>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_RMSNORM: return dispatch_rows<ROW_RMSNORM>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_SOFTMAX_VJP: return dispatch_rows<ROW_SOFTMAX_VJP>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_LAYERNORM_VJP: return dispatch_rows<ROW_LAYERNORM_VJP>(ca, cb, cy, n, cols, p, mask, s, fw);
+            case ROW_RMSNORM_VJP: return dispatch_rows<ROW_RMSNORM_VJP>(ca, cb, cy, n, cols, p, mask, s, fw);
+            default: return fail(MLXHIP_ERR_INVALID_ARGUMENT, "row op: unknown op %d", op);
+        }
+    });
 }
 
 int fibre_softmax(bool vjp, const float* a, const float* b, float* y, int64_t outer, int64_t dim,
