@@ -916,9 +916,13 @@ int gemm_impl(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, in
             // keeping at least 256 k (8 K tiles) per split. The 1000 x 777 x
             // 1531 product (56 tiles) runs 4 splits of 384 k on 224 CUs.
             int sp = 1;
-            // Packed operands: from 128 tiles on one workgroup per tile is faster (144
-            // tiles, K = 777: 24 us against 29 in two splits) and needs no partials.
-            if (cfg == 1 && path == 0 && !(padded && mid_tiles >= 128))
+            // Packed operands with a 16-bit C: from 128 tiles on one workgroup per
+            // tile is faster (144 tiles, K = 777: 24 us against 29 in two splits)
+            // and needs no partials. Its longer f32 sums are far below C's
+            // rounding (relative errors of 1601 x 1603 x 2047 before and after, bf16
+            // 1.65379587e-3 and ...588e-3, f16 2.06923247e-4 and ...378e-4), but an
+            // f32 C would show them.
+            if (cfg == 1 && path == 0 && !(padded && mid_tiles >= 128 && c_dtype != MLXHIP_DTYPE_F32))
                 while (sp < 8 && mid_tiles * sp < 256 && k / (2 * sp) >= 256) sp *= 2;
             // MLXHIP_GEMM16_SPLITS=s forces the split factor (1..8; tuning).
             if (const char* e = getenv("MLXHIP_GEMM16_SPLITS")) {

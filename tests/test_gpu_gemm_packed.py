@@ -49,3 +49,30 @@ def test_many_tiles_unaligned(m, n, k, batch, ta, tb, dtype, shift):
     for i in {0, batch - 1}:
         gemm_full_check(wide(np.ascontiguousarray(got[i, :, :n])), wide(a[i]), wide(b[i]), out=dtype,
                         what=f"{m}x{n}x{k} {dtype} slice {i}")
+
+
+def test_f32_result_of_packed_operands_keeps_its_k_splits():
+    """Slices too long for the kernels that read unaligned 16-bit rows (4 GiB:
+    1409 rows, 1.53 million elements apart) are packed with an f32 C too. 144
+    tiles: K is split as it is for the same product of aligned operands, and
+    the bits are that product's (its K padded with zeros)."""
+    m, n, k, kp = 1409, 1408, 1023, 1024
+    lda = (1 << 31) // (m - 1) + 2
+    lda += 1 - lda % 2
+    a, b = synth.bf16_bits(synth.normal(5, (m, k))), synth.bf16_bits(synth.normal(6, (k, n)))
+    da = hb.DeviceBuffer(((m - 1) * lda + k) * 2)
+    for i in range(m):
+        da.upload(a[i], offset=2 * i * lda)
+    db = hb.DeviceBuffer.from_array(b)
+    dc = hb.DeviceBuffer(m * n * 4)
+    hb.gemm(abi.BF16, abi.F32, False, False, m, n, k, da, lda, db, n, dc, n)
+    hb.synchronize()
+    got = dc.download(np.float32, m * n).reshape(m, n)
+    da.free()
+    ap, bp = np.zeros((m, kp), np.uint16), np.zeros((kp, n), np.uint16)
+    ap[:, :k], bp[:k] = a, b
+    da, db = hb.DeviceBuffer.from_array(ap), hb.DeviceBuffer.from_array(bp)
+    hb.gemm(abi.BF16, abi.F32, False, False, m, n, kp, da, kp, db, n, dc, n)
+    hb.synchronize()
+    np.testing.assert_array_equal(got.view(np.uint32), dc.download(np.uint32, m * n).reshape(m, n))
+    gemm_full_check(got, synth.bf16_to_f32(a), synth.bf16_to_f32(b), what="packed, f32 C")
