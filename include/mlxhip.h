@@ -363,11 +363,16 @@ int mlxhip_gemm(int32_t ab_dtype, int32_t c_dtype, int32_t trans_a, int32_t tran
  * of both operands, padded to multiples of 32) and split-K partials do not
  * fit that array runs on the direct f32 MFMA kernel instead, which needs
  * none (e.g. 4096^3 f32: 192 MiB of planes); its result is then within the
- * f32 bound but not bit-identical to mlxhip_gemm's. Any other product whose
+ * f32 bound but not bit-identical to mlxhip_gemm's. So does an unaligned
+ * product with a 16-bit C and 128 to 511 tiles of 128 x 128 whose padded copies
+ * do not fit: it runs on the kernel that reads unaligned rows (mlxhip_gemm
+ * packs up to 256 MiB), the same sums in another order before C's rounding.
+ * Any other product whose
  * workspace exceeds the array returns MLXHIP_ERR_INVALID_ARGUMENT (C is then
  * unchanged). Every call on one device
  * shares that device's array: calls that overlap on one device (several
- * streams or threads at once) race, so the caller serialises them. A call on
+ * streams or threads at once) race, so the caller serialises them (graph
+ * replays too: which products take scratch depends on size and alignment). A call on
  * a different stream than the previous call on that device, made while the
  * previous call's kernels have not finished, returns
  * MLXHIP_ERR_INVALID_ARGUMENT instead of racing (C unchanged); this check

@@ -255,7 +255,8 @@ def gemm_noalloc(ab_dtype: int, c_dtype: int, trans_a: bool, trans_b: bool, m: i
                  stream: int | None = None) -> None:
     """``gemm`` without any device allocation: its workspace comes from the
     library's fixed per-device scratch (``gemm_noalloc_scratch_bytes()``);
-    calls that overlap on one device race."""
+    calls that overlap on one device race. The bits are ``gemm``'s unless
+    that scratch is too small for the kernel (mlxhip.h)."""
     L = lib()
     abi.check(L.mlxhip_gemm_noalloc(ab_dtype, c_dtype, int(trans_a), int(trans_b), m, n, k, batch,
                                     _p(a), lda, stride_a, _p(b), ldb, stride_b, _p(c), ldc,

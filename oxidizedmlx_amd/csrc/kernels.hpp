@@ -285,9 +285,11 @@ bool gemm_wave_fits(int ab_dtype, int64_t m, int64_t n, int64_t k, int64_t batch
 int gemm_wave(int ab_dtype, int c_dtype, int ta, int tb, int64_t m, int64_t n, int64_t k, int64_t batch, const void* a,
               int64_t lda, int64_t sa, const void* b, int64_t ldb, int64_t sb, void* c, int64_t ldc, int64_t sc,
               const float* bias, bool aligned, hipStream_t s);
-// gemm with the same kernels and plan, its split-K partials and padded
-// operand copies taken from a fixed device array of
-// GEMM_NOALLOC_SCRATCH_BYTES instead of the memory pool: no allocation.
+// gemm with the same kernels and plan, its split-K partials, split-f32 planes
+// and padded operand copies taken from a fixed device array of
+// GEMM_NOALLOC_SCRATCH_BYTES instead of the memory pool: no allocation. Where
+// the planes, or the copies of 16-bit operands that another kernel can read as
+// they are, do not fit, that other kernel runs (not bit-identical to gemm).
 // Calls that overlap on one device share that array and race.
 constexpr size_t GEMM_NOALLOC_SCRATCH_BYTES = size_t(64) << 20;
 int gemm_noalloc(int ab_dtype, int c_dtype, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,

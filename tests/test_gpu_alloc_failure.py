@@ -5,15 +5,20 @@ in turn. Each failure must surface as MlxError::FfiFailed through the C ABI
 crash and no leak, and the library must work again once the hook is reset.
 The reference forces its error paths with bad shapes and parameters only
 (crates/mlx-core/tests/attention_golden.rs:259-302); running out of device
-memory is the failure a HIP backend adds."""
+memory is the failure a HIP backend adds. Workspace that only a faster kernel
+needs is no such point: without it the call runs on the other kernel (also
+test_gpu_prefill.py: a prompt taken a step per position)."""
 import ctypes as C
+import math
 
 import numpy as np
 import pytest
 
-from oxidizedmlx_amd import abi, nn
+from oxidizedmlx_amd import abi, nn, synth
 from oxidizedmlx_amd import backend as hb
 from oxidizedmlx_amd.opkind import OpKind, meta
+from parity import gemm_full_check
+from test_gpu_attention_vjp import f64_vjp
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip")]
 
@@ -118,3 +123,47 @@ def test_decoder_fails_cleanly_at_every_allocation(hook):
     built.close()
     hb.synchronize()
     assert before - free_device_bytes() < (64 << 20)
+
+
+def test_unaligned_product_without_room_for_its_copies(hook):
+    m, n, k = 1409, 1411, 65
+    a, b = synth.bf16_bits(synth.normal(1, (m, k))), synth.bf16_bits(synth.normal(2, (k, n)))
+    da, db, dc = hb.DeviceBuffer.from_array(a), hb.DeviceBuffer.from_array(b), hb.DeviceBuffer(m * n * 2)
+    s = hb.create_stream()  # without a workspace yet
+    try:
+        hook(0)
+        hb.gemm(abi.BF16, abi.BF16, False, False, m, n, k, da, k, db, n, dc, n, stream=s)
+        hook(-1)
+        hb.synchronize(s)
+    finally:
+        hb.destroy_stream(s)
+    got = synth.bf16_to_f32(dc.download(np.uint16, m * n)).reshape(m, n)
+    gemm_full_check(got, synth.bf16_to_f32(a), synth.bf16_to_f32(b), out="bf16", what="no room for copies")
+
+
+def test_sliced_gradient_without_room_for_its_partials(hook):
+    """The stream's workspace holds the row statistics of an earlier call, and
+    the slices' partials find no memory: the gradient runs whole. Its sums run
+    over up to 512 positions: sqrt(512) 2^-24 = 1.3e-6 of the largest value as a
+    random walk, allowed three times."""
+    h, t, scale = 1, 512, 1.0 / math.sqrt(64)
+    arrs = [synth.normal(20 + i, (h, t, 64)) for i in range(4)]
+    q, k, v, do = (hb.DeviceBuffer.from_array(x) for x in arrs)
+    o, dq, dk, dv = (hb.DeviceBuffer(arrs[0].nbytes) for _ in range(4))
+    big = [hb.DeviceBuffer(64 * 128 * 64 * 4) for _ in range(8)]  # 64 heads of 128: unsliced
+    for x in big[:5]:
+        x.upload(np.zeros(64 * 128 * 64, np.float32))
+    s = hb.create_stream()
+    try:
+        hb.attention_vjp(*big, 64, 128, 64, scale, True, stream=s)
+        hb.attention(q, k, v, o, h, t, t, 64, scale, True, stream=s)
+        hook(0)
+        hb.attention_vjp(q, k, v, o, do, dq, dk, dv, h, t, 64, scale, True, stream=s)
+        hook(-1)
+        hb.synchronize(s)
+    finally:
+        hb.destroy_stream(s)
+    for name, x, e in zip("qkv", (dq, dk, dv), f64_vjp(*arrs, scale, True)):
+        err = float(np.abs(x.download(np.float32, e.size).reshape(e.shape) - e).max())
+        print(f"  d{name}: {err:.3e}", flush=True)
+        assert err <= 4e-6 * float(np.abs(e).max())

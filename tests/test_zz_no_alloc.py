@@ -4,9 +4,11 @@ callers that cannot call hipMalloc) against mlxhip_gemm on the same operands.
 Both run the same kernels with the same split-K plan, so their outputs must
 agree bit for bit. Each case makes two calls in a row, the second on a
 smaller product, so the second call reads a fixed scratch that still holds
-the first call's partials. The cases cover the two workspace uses: split-K
-partials (f32 operands) and the zero-padded copies of unaligned operands
-(16-bit and f32, the latter then also split over K).
+the first call's partials. The cases cover the workspace uses: split-K
+partials and split-f32 planes (f32 operands), the zero-padded copies of
+unaligned 16-bit operands, and both at once in the f32 products whose K split
+follows packed copies; and products that take no scratch (the few-tile kernels
+read unaligned operands as they are).
 """
 import numpy as np
 import pytest
@@ -14,6 +16,7 @@ import pytest
 from oxidizedmlx_amd import abi
 from oxidizedmlx_amd import backend as hb
 from oxidizedmlx_amd import synth
+from parity import gemm_full_check
 
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("hip")]
 
@@ -43,19 +46,45 @@ def _run_both(m, n, k, dt, ld_pad, seed):
     return out
 
 
-@pytest.mark.parametrize("dt,ld_pad,shapes", [
-    # f32, aligned: split-K partials (8 x 1 MiB x 4 B, then 8 x 256 Ki x 4 B)
-    (F32, 0, [(1024, 1024, 2048), (512, 512, 1024)]),
-    # bf16, unaligned rows: both operands packed into scratch first
-    (BF16, 1, [(1000, 777, 1531), (300, 200, 333)]),
+@pytest.mark.parametrize("dt,ld_pad,shapes,scratch", [
+    # f32, aligned: split-f32 planes and their K partials; few tiles: no scratch
+    (F32, 0, [(1024, 1024, 2048), (512, 512, 1024)], [True, False]),
+    # bf16, unaligned rows, fewer than 128 tiles: read as they are
+    (BF16, 1, [(1000, 777, 1531), (300, 200, 333)], [False, False]),
+    # f32, unaligned rows, few tiles: read as they are
+    (F32, 1, [(513, 300, 1999), (129, 65, 700)], [False, False]),
+    # More than 1024 tiles of 64 x 64, fewer than 256 rows (no planes). f32,
+    # aligned: partials of a K split in two
+    (F32, 0, [(200, 16448, 512), (196, 16388, 512)], [True, True]),
     # f32, unaligned rows: packed copies, then split-K partials after them
-    (F32, 1, [(513, 300, 1999), (129, 65, 700)]),
-], ids=["f32_splitk", "bf16_packed", "f32_packed_splitk"])
-def test_noalloc_matches_gemm_on_two_calls(dt, ld_pad, shapes):
+    (F32, 1, [(200, 16401, 513), (199, 16397, 512)], [True, True]),
+    # bf16, unaligned rows, from 128 tiles of 256 x 256: both operands packed
+    (BF16, 1, [(2900, 2819, 65), (2818, 2818, 41)], [True, True]),
+], ids=["f32_planes", "bf16_as_it_is", "f32_as_it_is", "f32_splitk", "f32_packed_splitk", "bf16_packed"])
+def test_noalloc_matches_gemm_on_two_calls(dt, ld_pad, shapes, scratch):
     for i, (m, n, k) in enumerate(shapes):
         print(f"noalloc case dt={dt} pad={ld_pad} call {i}: {m}x{n}x{k}", flush=True)
         ref, got = _run_both(m, n, k, dt, ld_pad, seed=17 + i)
         assert np.array_equal(ref, got), f"call {i} {m}x{n}x{k}: {int((ref != got).sum())} elements differ"
+        assert _takes_workspace(m, n, k, dt, ld_pad) == scratch[i]
+
+
+def _takes_workspace(m, n, k, dt, ld_pad):
+    """Whether mlxhip_gemm fails on a new stream without memory for workspace."""
+    L = abi.load_library()
+    es = 2 if dt == BF16 else 4
+    bufs = [hb.DeviceBuffer(m * (k + ld_pad) * es), hb.DeviceBuffer(k * (n + ld_pad) * es), hb.DeviceBuffer(m * n * 4)]
+    s = hb.create_stream()
+    L.mlxhip_debug_fail_allocations(0)
+    try:
+        hb.gemm(dt, F32, False, False, m, n, k, bufs[0], k + ld_pad, bufs[1], n + ld_pad, bufs[2], n, stream=s)
+        hb.synchronize(s)
+        return False
+    except abi.FfiFailed:
+        return True
+    finally:
+        L.mlxhip_debug_fail_allocations(-1)
+        hb.destroy_stream(s)
 
 
 def test_noalloc_rejects_products_beyond_its_scratch():
@@ -95,6 +124,23 @@ def test_noalloc_f32_planes_beyond_scratch_take_the_direct_kernel():
     bound = (k * np.finfo(np.float32).eps) * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64))
     err = np.abs(got - ref)
     assert np.all(err <= bound + 1e-30), float((err / np.maximum(bound, 1e-30)).max())
+
+
+def test_noalloc_copies_beyond_scratch_take_the_unpacked_kernel():
+    """An unaligned bf16 product of 144 tiles whose padded copies (66 MiB) exceed
+    the scratch runs on the kernel that reads its rows as they are; mlxhip_gemm
+    packs it. Both within the bound of one rounding to bf16."""
+    m, n, k = 1500, 1501, 11501
+    a, b = synth.bf16_bits(synth.normal(33, (m, k))), synth.bf16_bits(synth.normal(34, (k, n)))
+    da, db = hb.DeviceBuffer.from_array(a), hb.DeviceBuffer.from_array(b)
+    print(f"noalloc bf16 unpacked: {m}x{n}x{k}", flush=True)
+    for fn in (hb.gemm, hb.gemm_noalloc):
+        dc = hb.DeviceBuffer(m * n * 2)
+        fn(BF16, BF16, False, False, m, n, k, da, k, db, n, dc, n)
+        hb.synchronize()
+        got = synth.bf16_to_f32(dc.download(np.uint16, m * n)).reshape(m, n)
+        for rows in (slice(0, 40), slice(m - 40, m)):
+            gemm_full_check(got[rows], synth.bf16_to_f32(a[rows]), synth.bf16_to_f32(b), out="bf16", what=fn.__name__)
 
 
 def test_noalloc_refuses_another_stream_while_the_scratch_is_busy():
