@@ -77,9 +77,9 @@ int eval_matmul_bias(const mlxhip_input_t* inputs, const mlxhip_meta_t& out_meta
 
 // Copies `bytes` of device memory into pageable host memory after everything
 // queued on `s`; returns when they have arrived. Large copies go through
-// pinned stages by several threads (host_copy.cpp). A stage is kept for the
-// next copy between host_copy_retain and the matching host_copy_release
-// (every Stream and decoder holds one).
+// pinned slots by several threads (host_copy.cpp), which are kept for later
+// copies between host_copy_retain and the matching host_copy_release (every
+// Stream and decoder holds one).
 int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s);
 void host_copy_retain();
 void host_copy_release();

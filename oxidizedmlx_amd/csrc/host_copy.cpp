@@ -4,24 +4,26 @@
 //
 // hipMemcpy into pageable memory goes through the runtime's staging with one
 // thread, which also takes the page faults of a fresh destination: 17 GB/s on
-// memory that is already mapped, about 10 GB/s on new memory, where the link
+// memory that is already mapped, about 4 GB/s on new memory, where the link
 // carries 55 GB/s into pinned memory. Here several threads each move chunks
-// through a pinned slot of their own, so one chunk's copy by the CPU (and its
-// page faults) runs beside the others' transfers. Into a new numpy array:
-// 64 MiB 6.3 -> 1.9 ms, 16 MiB 0.94 -> 0.60 ms, 4 MiB 246 -> 205 us, 1 MiB
-// 430 -> 77 us (one thread).
+// through a pinned slot of their own (host_slots.hpp), so one chunk's copy by
+// the CPU (and its page faults) runs beside the others' transfers.
+// us through the runtime's way / here with kept slots, into new pages (and
+// into mapped ones): 128 KiB 92 / 30 (17 / 16), 1 MiB 290 / 215 (65 / 61), 2 MiB
+// 580 / 430 (121 / 113), 4 MiB 1150 / 920 (240 / 203), 16 MiB 4550 / 3600 (950 /
+// 580), 64 MiB 18100 / 14200 (3900 / 1820).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <mutex>
 #include <system_error>
 #include <thread>
 #include <vector>
 
 #include "backend.hpp"
 #include "common.hpp"
+#include "host_slots.hpp"
 
 namespace mlxhip {
 namespace {
@@ -32,94 +34,84 @@ constexpr size_t HUGE = size_t(2) << 20;  // a transparent huge page of the dest
 constexpr size_t CHUNK = HUGE;
 constexpr size_t PAGE = 4096;
 constexpr int MAX_WORKERS = 8;
-constexpr size_t STAGE_BYTES = CHUNK * MAX_WORKERS;
 constexpr size_t MIN_BYTES = size_t(128) << 10;  // below, the runtime's own staging is as fast
+// Slots that a copy of several chunks needs to be ahead of the runtime's way.
+constexpr int MIN_WORKERS = 4;
 
-// Pinned stages kept for the next copy while any Stream or decoder lives (at
-// most MAX_KEPT; concurrent copies beyond that allocate and free their own).
-constexpr size_t MAX_KEPT = 2;
-std::mutex g_mu;
-std::vector<char*> g_kept;
-int g_owners = 0;
-
-char* take_stage() {
-    {
-        std::lock_guard<std::mutex> g(g_mu);
-        if (!g_kept.empty()) {
-            char* p = g_kept.back();
-            g_kept.pop_back();
-            return p;
-        }
-    }
+char* pin_slot() {
+    // Not a stream operation: allowed while another thread's stream is captured.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
     void* p = nullptr;
-    if (hipHostMalloc(&p, STAGE_BYTES, hipHostMallocPortable) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    return static_cast<char*>(p);
+    const hipError_t e = hipHostMalloc(&p, CHUNK, hipHostMallocPortable);
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return static_cast<char*>(p);
+    (void)hipGetLastError();
+    return nullptr;
 }
 
-void give_stage(char* p) {
-    {
-        std::lock_guard<std::mutex> g(g_mu);
-        if (g_owners > 0 && g_kept.size() < MAX_KEPT) {
-            g_kept.push_back(p);
-            return;
-        }
-    }
-    (void)hipHostFree(p);
+void unpin_slot(char* p) { (void)hipHostFree(p); }
+
+HostSlots& slots() {
+    static HostSlots* p = new HostSlots(pin_slot, unpin_slot);  // never destroyed: outlives late frees at exit
+    return *p;
+}
+
+// Faults the pages of [p, p + n) in (all of them are written afterwards).
+void touch(char* p, size_t n) {
+    for (size_t i = 0; i < n; i += PAGE) *static_cast<volatile char*>(p + i) = 0;
 }
 
 }  // namespace
 
-void host_copy_retain() {
-    std::lock_guard<std::mutex> g(g_mu);
-    ++g_owners;
-}
-
-void host_copy_release() {
-    std::vector<char*> drop;
-    {
-        std::lock_guard<std::mutex> g(g_mu);
-        if (--g_owners == 0) drop.swap(g_kept);
-    }
-    for (char* p : drop) (void)hipHostFree(p);
-}
+void host_copy_retain() { slots().retain(); }
+void host_copy_release() { slots().release(); }
 
 int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    char* stage = bytes >= MIN_BYTES ? take_stage() : nullptr;
-    if (!stage) {
-        MLXHIP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-        MLXHIP_HIP(hipStreamSynchronize(s));
-        return MLXHIP_OK;
-    }
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    char* to = static_cast<char*>(dst);
-    const char* from = static_cast<const char*>(src);
     // Chunks end at 2 MiB boundaries of the destination, so that no two threads
     // fault the same huge page.
     const size_t head = bytes <= CHUNK ? bytes : CHUNK - reinterpret_cast<uintptr_t>(dst) % HUGE;
     const int chunks = 1 + (int)((bytes - head + CHUNK - 1) / CHUNK);
+    char* slot[MAX_WORKERS];
+    int workers = 0;
+    if (bytes >= MIN_BYTES) {
+        static const int cpus = (int)std::thread::hardware_concurrency();
+        const int most = std::max(1, std::min({chunks, MAX_WORKERS, cpus / 2}));
+        workers = slots().take(bytes, most, std::min(most, MIN_WORKERS), slot);
+    }
+    if (workers == 0) {
+        MLXHIP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        MLXHIP_HIP(hipStreamSynchronize(s));
+        return MLXHIP_OK;
+    }
+    char* to = static_cast<char*>(dst);
+    const char* from = static_cast<const char*>(src);
+    if (chunks == 1) {
+        hipError_t e = hipMemcpyAsync(slot[0], from, bytes, hipMemcpyDeviceToHost, s);
+        touch(to, bytes);  // while the transfer runs
+        const hipError_t es = hipStreamSynchronize(s);
+        if (e == hipSuccess) e = es;
+        if (e == hipSuccess) std::memcpy(to, slot[0], bytes);
+        slots().give(slot, 1);
+        return e == hipSuccess ? MLXHIP_OK : hip_fail(e, "copy to host");
+    }
+    int dev = 0;
+    (void)hipGetDevice(&dev);
     std::atomic<int> next{0}, error{(int)hipSuccess};
     auto work = [&](int w) noexcept {
         hipEvent_t ev = nullptr;
         hipError_t e = hipSetDevice(dev);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-        char* slot = stage + (size_t)w * CHUNK;
         while (e == hipSuccess && error.load() == (int)hipSuccess) {
             const int c = next.fetch_add(1);
             if (c >= chunks) break;
             const size_t lo = c == 0 ? 0 : head + (size_t)(c - 1) * CHUNK;
             const size_t n = std::min(bytes, head + (size_t)c * CHUNK) - lo;
-            e = hipMemcpyAsync(slot, from + lo, n, hipMemcpyDeviceToHost, s);
+            e = hipMemcpyAsync(slot[w], from + lo, n, hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipEventRecord(ev, s);
-            // Fault the chunk's pages in while its transfer runs (all of it is
-            // written below).
-            if (e == hipSuccess)
-                for (size_t i = 0; i < n; i += PAGE) *static_cast<volatile char*>(to + lo + i) = 0;
+            if (e == hipSuccess) touch(to + lo, n);  // while its transfer runs
             if (e == hipSuccess) e = hipEventSynchronize(ev);
-            if (e == hipSuccess) std::memcpy(to + lo, slot, n);
+            if (e == hipSuccess) std::memcpy(to + lo, slot[w], n);
         }
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -127,8 +119,6 @@ int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
         }
         if (ev) (void)hipEventDestroy(ev);
     };
-    const int cpus = (int)std::thread::hardware_concurrency();
-    const int workers = std::max(1, std::min({chunks, MAX_WORKERS, cpus / 2}));
     std::vector<std::thread> threads;
     try {
         threads.reserve((size_t)workers);
@@ -139,9 +129,9 @@ int copy_to_host(void* dst, const void* src, size_t bytes, hipStream_t s) {
     work(0);
     for (std::thread& t : threads) t.join();
     const hipError_t e = (hipError_t)error.load();
-    // A failed copy may leave transfers queued into the stage.
+    // A failed copy may leave transfers queued into the slots.
     if (e != hipSuccess) (void)hipStreamSynchronize(s);
-    give_stage(stage);
+    slots().give(slot, workers);
     return e == hipSuccess ? MLXHIP_OK : hip_fail(e, "copy to host");
 }
 

@@ -1,6 +1,11 @@
 """Large results into pageable memory (csrc/host_copy.cpp): sizes around the
 line (128 KiB) and the chunks (2 MiB of the destination), destinations at any
-alignment, several streams at once from several threads."""
+alignment, several streams at once from several threads; through the pinned
+slots, which a stream that stays open has earned (csrc/host_slots.hpp,
+test_host_slots.py), and the runtime's way."""
+import os
+import subprocess
+import sys
 import threading
 
 import numpy as np
@@ -22,9 +27,20 @@ def negated(st, n, seed):
     return x, node
 
 
+@pytest.fixture(scope="module")
+def owner():
+    """A stream that has copied 576 MiB: every slot is earned while it lives."""
+    st = HipStream()
+    x, node = negated(st, 64 * MIB, 1)
+    for _ in range(9):
+        np.testing.assert_array_equal(st.get_buffer(node), -x)
+    yield st
+    st.close()
+
+
 @pytest.mark.parametrize("n", [(1 << 15) - 1, 1 << 15, 2 * MIB, 2 * MIB + 1, 4 * MIB - 1, 4 * MIB, 21 * MIB - 7])
 @pytest.mark.parametrize("offset", [0, 1, 100003])
-def test_sizes_and_alignments(n, offset):
+def test_sizes_and_alignments(owner, n, offset):
     st = HipStream()
     x, node = negated(st, n, n + offset)
     out = np.full(offset + n + 1, 7.0, np.float32)
@@ -34,7 +50,7 @@ def test_sizes_and_alignments(n, offset):
     st.close()
 
 
-def test_threads_with_streams_of_their_own():
+def test_threads_with_streams_of_their_own(owner):
     bad = []
 
     def work(seed):
@@ -51,3 +67,23 @@ def test_threads_with_streams_of_their_own():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_a_first_fetch_goes_the_runtimes_way():
+    """In a process of its own: the first copies have no slots yet."""
+    code = """
+import numpy as np
+from oxidizedmlx_amd.backend import HipStream
+from oxidizedmlx_amd.opkind import OpKind, meta
+for n in (1 << 15, (1 << 19) + 3, 5 << 18):
+    st = HipStream()
+    x = np.arange(n, dtype=np.float32)
+    node = st.add_op(OpKind.Neg, [st.add_constant(x, meta([n]))], meta([n]))
+    st.eval(node)
+    assert np.array_equal(st.get_buffer(node), -x)
+    st.close()
+print("ok")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.stdout.strip() == "ok", r.stdout + r.stderr
