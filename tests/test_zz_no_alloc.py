@@ -10,6 +10,8 @@ unaligned 16-bit operands, and both at once in the f32 products whose K split
 follows packed copies; and products that take no scratch (the few-tile kernels
 read unaligned operands as they are).
 """
+import gc
+
 import numpy as np
 import pytest
 
@@ -162,6 +164,7 @@ def test_noalloc_refuses_another_stream_while_the_scratch_is_busy():
         c2 = hb.DeviceBuffer.from_array(sentinel)
         ref = hb.DeviceBuffer(m * nn * 4)
         hb.synchronize()
+        gc.collect()  # a collection of a long session's objects takes longer than the queued work
         # ~3 ms of 4096^3 bf16 products ahead of stream 1's noalloc call.
         for _ in range(24):
             hb.gemm(BF16, BF16, False, False, n, n, n, busy[0], n, busy[1], n, busy_c, n, stream=s1)
