@@ -23,8 +23,10 @@
 //   accumulates dK and dV.
 //   With few heads both are sliced over more workgroups (attention_vjp).
 //
-// Bound by the f32 matrix rate (64 heads x 1024, causal: 36.5 GFLOP over the
-// visible blocks in 327 us, 112 TFLOP/s; a large f32 product reaches 138).
+// Bound by the rate of the f32 MFMA (64 heads x 1024, causal: 36.5 GFLOP over
+// the visible blocks in 327 us, 112 TFLOP/s; a large f32 product reaches 138 on
+// it). The forward's form, six products of bf16 planes, has a higher bound and
+// was not written here. The dK/dV kernel spills 11 VGPRs of a lane.
 // Products are v_mfma_f32_32x32x2_f32 (exact f32 products, f32 sums). A
 // workgroup's 4 waves each own a 32 x 32 tile of the 64 x 64 block: wave w
 // takes query half qh = w & 1 and key half kh = w >> 1. For an MFMA lane l,
