@@ -5,8 +5,6 @@ copies, given back with the last owner, and counted right when pinning fails
 or many threads take them at once."""
 import subprocess
 
-import pytest
-
 from oxidizedmlx_amd import build
 
 PROGRAM = r"""
@@ -102,10 +100,9 @@ int main() {
 """
 
 
-@pytest.mark.parametrize("flags", [[], ["-fsanitize=thread", "-g"]], ids=["plain", "tsan"])
-def test_slots_are_earned_bounded_and_given_back(tmp_path, flags):
+def test_slots_are_earned_bounded_and_given_back(tmp_path):
     (tmp_path / "p.cpp").write_text(PROGRAM)
-    subprocess.run(["g++", "-std=c++17", "-O1", *flags, "-I", build.CSRC, "-o", str(tmp_path / "p"), str(tmp_path / "p.cpp"),
-                    "-pthread"], check=True)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", build.CSRC, "-o", str(tmp_path / "p"), str(tmp_path / "p.cpp"), "-pthread"],
+                   check=True)
     r = subprocess.run([str(tmp_path / "p")], capture_output=True, text=True, timeout=120)
     assert r.stdout.strip() == "ok" and r.returncode == 0, r.stdout + r.stderr
